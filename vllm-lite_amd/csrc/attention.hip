@@ -56,6 +56,10 @@ constexpr int kPlanThreads = 256;
 constexpr int kMaxHeadDim = 256;
 constexpr int kSplitMaxQ = 16;  // only sequences with <= this many queries split their context
 constexpr int kPart0 = 64;  // first partition length tried by the planner
+// fp32 tile items of longer query chunks are cut over the context too, into
+// about this many items per compute unit, but not below kChunkPart keys each
+constexpr int kChunkItemsPerCu = 3;
+constexpr int kChunkPart = 256;
 constexpr float kLog2e = 1.4426950408889634f;
 
 // bandwidth-kernel shape
@@ -266,8 +270,15 @@ struct SeqWork {
 // generic kernel.
 __device__ __forceinline__ bool is_bw(int q, int c, bool fast) { return fast && q == 1 && c > 0; }
 
-__device__ __forceinline__ SeqWork seq_work(int q, int c, int P, int R, int H, int Hkv, bool fast,
-                                            bool tile, bool wide) {
+// P2 > 0: fp32 tile chunks (q > kSplitMaxQ) are split too, into equal parts
+// of about P2 keys (whole key tiles; the tile kernel derives the length from
+// the part count, chunk_part_len).
+__device__ __forceinline__ int chunk_part_len(int c, int np) {
+  return cdiv(cdiv(c, kTileKeys), np) * kTileKeys;
+}
+
+__device__ __forceinline__ SeqWork seq_work(int q, int c, int P, int P2, int R, int H, int Hkv,
+                                            bool fast, bool tile, bool wide) {
   SeqWork w;
   const bool live = q > 0 && c > 0;
   const bool bw = is_bw(q, c, fast);
@@ -278,6 +289,8 @@ __device__ __forceinline__ SeqWork seq_work(int q, int c, int P, int R, int H, i
     w.tail = (c % R) != 0;
   } else {
     w.np = (q > 0 && q <= kSplitMaxQ && c > P) ? (c + P - 1) / P : 1;
+    if (tl && !wide && q > kSplitMaxQ && P2 > 0 && c > P2)
+      w.np = cdiv(c, chunk_part_len(c, cdiv(c, P2)));  // no part is empty
     w.full = w.tail = 0;
   }
   const bool wd = tl && wide && q > kSplitMaxQ;  // never split (np == 1)
@@ -412,14 +425,14 @@ template <bool kCached>
 __global__ void __launch_bounds__(kPlanThreads) plan_kernel(
     const int32_t* __restrict__ seq_lens, const int32_t* __restrict__ qsl, int S, int H, int Hkv,
     bool fast, bool tile, bool wide, int64_t cap_rows, int target_items, int tile_target,
-    int32_t* __restrict__ hdr, int32_t* __restrict__ gen_off,
+    int chunk_target, int32_t* __restrict__ hdr, int32_t* __restrict__ gen_off,
     int32_t* __restrict__ tile_off, int32_t* __restrict__ nparts,
     int32_t* __restrict__ split_base, int32_t* __restrict__ wide_off,
     int32_t* __restrict__ cmb_seq, int32_t* __restrict__ wide_seq,
     int32_t* __restrict__ tail_seq, int32_t* __restrict__ tail_off, int4* __restrict__ desc,
     float2* __restrict__ ml) {
   constexpr int kWaves = kPlanThreads / 64;
-  __shared__ unsigned long long red0[kWaves][2], red1[2][kWaves][1];
+  __shared__ unsigned long long red0[kWaves][3], red1[2][kWaves][1];
   __shared__ int hist[kTailBuckets], whist[kTailBuckets], thist[kTailBuckets];
   // with at most kPlanLdsSeqs sequences, the item counts of the 32-row list
   // and of the second 16-row list by position, so that their offsets need no
@@ -433,16 +446,16 @@ __global__ void __launch_bounds__(kPlanThreads) plan_kernel(
   // 0. range length from the decode tokens and the target item count; the
   // same for the partition length of the splittable multi-query sequences
   // (at most kSplitMaxQ queries), counted in (KV head, 64-row block) units
-  int R = 64, P = kPart0;
-  bool lpt;  // the 16-row items in two lists, the last partitions longest first
+  int R = 64, P = kPart0, P2 = 0;
+  bool lpt;  // 16-row items (or bf16 ones' last partitions) handed out longest first
   {
     const int rep = H / Hkv;
-    unsigned long long v[2] = {0, 0};
+    unsigned long long v[3] = {0, 0, 0};
     ch.each(qsl, seq_lens, [&](int, int q, int c) {
       if (is_bw(q, c, fast))
         v[0] += (unsigned long long)c;
-      else if (tile && q > 0 && q <= kSplitMaxQ && c > 0)
-        v[1] += (unsigned long long)c * cdiv(q * rep, kTileRows);
+      else if (tile && q > 0 && c > 0)
+        v[q <= kSplitMaxQ ? 1 : 2] += (unsigned long long)c * cdiv(q * rep, kTileRows);
     });
     plan_sum(v, red0);  // its barrier also orders the histogram clearing
     while (R < kRangeMax && v[0] * (unsigned long long)Hkv >
@@ -451,18 +464,25 @@ __global__ void __launch_bounds__(kPlanThreads) plan_kernel(
     while (P < (1 << 20) && v[1] * (unsigned long long)Hkv >
                                 (unsigned long long)max(tile_target, 1) * (unsigned long long)P)
       P *= 2;
-    lpt = wide && v[1] > 0;  // bf16 16-row items (short queries over split contexts)
+    if (tile && !wide && v[2] > 0) {
+      const unsigned long long len = v[2] * (unsigned long long)Hkv / max(chunk_target, 1);
+      P2 = (int)min((unsigned long long)(1 << 29), max((unsigned long long)kChunkPart, len));
+    }
+    lpt = wide ? v[1] > 0 : v[1] + v[2] > 0;
   }
   // 1. double P and R until the split partials fit (every thread holds the
   // same sums, so all take the same branch)
   for (int it = 0;; ++it) {
     unsigned long long need[1] = {0};
     ch.each(qsl, seq_lens, [&](int, int q, int c) {
-      need[0] += seq_work(q, c, P, R, H, Hkv, fast, tile, wide).rows;
+      need[0] += seq_work(q, c, P, P2, R, H, Hkv, fast, tile, wide).rows;
     });
     plan_sum(need, red1[it & 1]);
     if (need[0] <= (unsigned long long)cap_rows || (P >= (1 << 29) && R >= (1 << 29))) break;
-    P = min(P * 2, 1 << 29), R = min(R * 2, 1 << 29);
+    if (P2 > 0)
+      P2 = 0;  // the chunks' partials do not fit beside the others: leave them whole
+    else
+      P = min(P * 2, 1 << 29), R = min(R * 2, 1 << 29);
   }
   // 2. offsets
   // tail ranges are bucketed by their length in blocks, longest first
@@ -484,19 +504,23 @@ __global__ void __launch_bounds__(kPlanThreads) plan_kernel(
   // order; the second the last partitions' items, sequences ordered by that
   // partition's length in 64-key tiles, descending (sequences without such
   // items in the last bucket), so that a launch ends on its shortest items.
-  // Otherwise (fp32 items: short contexts, tiny items) the first list holds
-  // them all, in sequence order.
+  // fp32 items are all in the second list, sequences ordered by the length of
+  // their partitions, descending: a batch mixes chunk items of many key tiles
+  // (32 fp32 MFMA cycles per 16 x 16 x 4 product) with one-tile decode items,
+  // and the chunk items have to start first.
   auto split_items = [&](const SeqWork& w) -> int64_t {
-    return !lpt ? w.tile : w.tile > 0 ? w.tile / w.np * (w.np - 1) : 0;
+    return !lpt ? w.tile : w.tile > 0 && wide ? w.tile / w.np * (w.np - 1) : 0;
   };
-  auto last_key = [&](int c, const SeqWork& w) {
+  auto last_key = [&](int q, int c, const SeqWork& w) {
     if (w.tile == 0 || !lpt) return kTailBuckets - 1;
-    const int64_t last = (int64_t)c - (int64_t)(w.np - 1) * P;  // 1 .. P keys (all of c unsplit)
+    const int64_t last = wide ? (int64_t)c - (int64_t)(w.np - 1) * P  // 1 .. P keys (all of c unsplit)
+                         : q > kSplitMaxQ ? chunk_part_len(c, w.np)
+                                          : min(c, P);
     return kTailBuckets - 2 - (int)min<int64_t>(kTailBuckets - 2, cdiv64(last, kTileKeys) - 1);
   };
   int64_t f = 0, g = 0, r = 0, x = 0, xs = 0, tl = 0, wd = 0, cm = 0;
   ch.each(qsl, seq_lens, [&](int, int q, int c) {
-    const SeqWork w = seq_work(q, c, P, R, H, Hkv, fast, tile, wide);
+    const SeqWork w = seq_work(q, c, P, P2, R, H, Hkv, fast, tile, wide);
     f += w.full, g += w.gen, r += w.rows, x += w.tile, tl += w.tail, wd += w.wide;
     xs += split_items(w);
     cm += w.np > 1 && w.gen > 0;  // the combine kernel merges only the generic kernel's splits
@@ -505,7 +529,7 @@ __global__ void __launch_bounds__(kPlanThreads) plan_kernel(
       bucket_add<false>(hist, key, __builtin_amdgcn_readfirstlane(key));
     }
     bucket_add<false>(whist, wide_key(c, w.wide > 0), kTailBuckets - 1);
-    if (lpt) bucket_add<false>(thist, last_key(c, w), kTailBuckets - 1);
+    if (lpt) bucket_add<false>(thist, last_key(q, c, w), kTailBuckets - 1);
   });
   __syncthreads();
   // the thread's buckets: their counts, summed, join the same scan as the
@@ -533,7 +557,7 @@ __global__ void __launch_bounds__(kPlanThreads) plan_kernel(
   }
   __syncthreads();
   ch.each(qsl, seq_lens, [&](int i, int q, int c) {
-    const SeqWork w = seq_work(q, c, P, R, H, Hkv, fast, tile, wide);
+    const SeqWork w = seq_work(q, c, P, P2, R, H, Hkv, fast, tile, wide);
     const int qs = qsl[i];
     for (int k = 0; k < w.full; ++k) desc[fo + k] = make_int4(i, k, c, qs);
     gen_off[i] = (int32_t)go;
@@ -544,7 +568,7 @@ __global__ void __launch_bounds__(kPlanThreads) plan_kernel(
       if (S <= kPlanLdsSeqs) wcnt[p] = (int)w.wide;
     }
     if (lpt) {
-      const int p = bucket_add<true>(thist, last_key(c, w), kTailBuckets - 1);
+      const int p = bucket_add<true>(thist, last_key(q, c, w), kTailBuckets - 1);
       tail_seq[p] = i;
       if (S <= kPlanLdsSeqs) tcnt[p] = (int)(w.tile - split_items(w));
     }
@@ -570,12 +594,12 @@ __global__ void __launch_bounds__(kPlanThreads) plan_kernel(
     auto wide_items = [&](int p) -> int64_t {
       if (S <= kPlanLdsSeqs) return wcnt[p];
       const int i = wide_seq[p];
-      return seq_work(qsl[i + 1] - qsl[i], seq_lens[i], P, R, H, Hkv, fast, tile, wide).wide;
+      return seq_work(qsl[i + 1] - qsl[i], seq_lens[i], P, P2, R, H, Hkv, fast, tile, wide).wide;
     };
     auto last_items = [&](int p) -> int64_t {
       if (S <= kPlanLdsSeqs) return tcnt[p];
       const int i = tail_seq[p];
-      const SeqWork w = seq_work(qsl[i + 1] - qsl[i], seq_lens[i], P, R, H, Hkv, fast, tile, wide);
+      const SeqWork w = seq_work(qsl[i + 1] - qsl[i], seq_lens[i], P, P2, R, H, Hkv, fast, tile, wide);
       return w.tile - split_items(w);
     };
     int64_t mw = 0, mt = 0;
@@ -744,11 +768,23 @@ __global__ void __launch_bounds__(64) attend_generic_kernel(
 //                                      + e - 4, and V^T is read in that order.
 // bf16 uses v_mfma_f32_16x16x32_bf16 (P rounded to bf16, fp32 accumulation);
 // fp32 uses v_mfma_f32_16x16x4f32, so fp32 inputs keep fp32 products.
+//
+// The fp32 items are bound by the matrix pipe: a 64-key tile of 16 rows at
+// head_dim 64 is 128 products of 32 cycles (1.7 us at 2.4 GHz), against 0.9 us
+// for its softmax, staging and barriers. One 16-byte LDS read feeds 4 products
+// of QK^T or PV (4-byte reads at an odd row stride met 4-way bank conflicts);
+// items start longest first, and chunks are cut over the context into about
+// 3 items per compute unit, so that one long row block does not set the time.
+// 24 decodes + 5 chunks of 300-500 queries, 8 heads of 64: 208 us before, of it
+// 201 in this kernel; 160 with the wide reads, 126 with the order and the cut,
+// 101 with the 16-byte merge (merge_tile_rows).
 
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
+typedef float f32x2_t __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
 
 // 16-byte global load as a native vector (a uint4 struct copy can become an
 // aggregate memcpy that keeps a register array in scratch memory)
@@ -756,34 +792,49 @@ __device__ __forceinline__ uint4 load16(const void* p) {
   return __builtin_bit_cast(uint4, *reinterpret_cast<const u32x4_t*>(p));
 }
 
-// 4 consecutive cache elements as the bits of 4 fp32 values: fp32 as they
-// are, bf16 and FP8 E4M3 widened (exactly) for the fp32 tile path
-__device__ __forceinline__ uint4 load4_as_f32(const float* p) { return load16(p); }
-__device__ __forceinline__ uint4 load4_as_f32(const uint16_t* p) {
-  const uint2 w = *reinterpret_cast<const uint2*>(p);
-  return make_uint4(w.x << 16, w.x & 0xffff0000u, w.y << 16, w.y & 0xffff0000u);
-}
-__device__ __forceinline__ uint4 load4_as_f32(const uint8_t* p) {
-  float r[4];
-  e4m3x4_to_f32(*reinterpret_cast<const uint32_t*>(p), r);
-  return make_uint4(__float_as_uint(r[0]), __float_as_uint(r[1]), __float_as_uint(r[2]),
-                    __float_as_uint(r[3]));
-}
+// 4 consecutive cache elements for the fp32 tile path: loaded as they are
+// (16, 8 or 4 bytes), widened to fp32 (exactly) when they are staged in LDS,
+// so that a tile in flight holds no more registers than its bytes
+template <typename TKV>
+struct Cache4;
+template <>
+struct Cache4<float> {
+  typedef u32x4_t Raw;
+  static __device__ __forceinline__ f32x4_t widen(Raw r) { return __builtin_bit_cast(f32x4_t, r); }
+};
+template <>
+struct Cache4<uint16_t> {
+  typedef u32x2_t Raw;
+  static __device__ __forceinline__ f32x4_t widen(Raw r) {
+    const u32x4_t w = {r[0] << 16, r[0] & 0xffff0000u, r[1] << 16, r[1] & 0xffff0000u};
+    return __builtin_bit_cast(f32x4_t, w);
+  }
+};
+template <>
+struct Cache4<uint8_t> {
+  typedef uint32_t Raw;
+  static __device__ __forceinline__ f32x4_t widen(Raw r) {
+    float f[4];
+    e4m3x4_to_f32(r, f);
+    return (f32x4_t){f[0], f[1], f[2], f[3]};
+  }
+};
 
-// The same for the K / V bytes of a tile item: a non-temporal (streaming)
-// load when no other item reads them (a sequence whose rows fit one item:
-// spec-verify and short chunks; measured 950 -> 870 us on the 64 x 5 verify
-// batch), an ordinary one when the sequence's other row blocks re-read them
-// from the cache (long prefill chunks: streaming loads there measured 281 ->
-// 298 us)
-// kStream: a non-temporal load (data read once). A compile-time choice: a
-// runtime one puts every load in a branch of its own, and the compiler then
-// cannot issue a tile's loads (and the block-id loads they need) together.
-template <bool kStream>
-__device__ __forceinline__ uint4 load16_kv(const void* p) {
-  if constexpr (kStream)
-    return __builtin_bit_cast(uint4, __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(p)));
-  return load16(p);
+// K / V cache bytes of a tile item (a Raw of them), by a non-temporal
+// (streaming) load or not. The choice is a compile-time one: a runtime one
+// puts every load in a branch of its own, and the compiler then cannot issue
+// a tile's loads (and the block-id loads they need) together.
+template <bool kStream, typename Raw>
+__device__ __forceinline__ Raw load_kv(const void* p) {
+  if constexpr (std::is_same<Raw, uint4>::value) {
+    if constexpr (kStream)
+      return __builtin_bit_cast(uint4,
+                                __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(p)));
+    return load16(p);
+  } else {
+    if constexpr (kStream) return __builtin_nontemporal_load(reinterpret_cast<const Raw*>(p));
+    return *reinterpret_cast<const Raw*>(p);
+  }
 }
 
 // One K/V tile in LDS. RW (rows per wavefront) sets the V^T row stride: the
@@ -802,6 +853,7 @@ struct alignas(16) TileLds<uint16_t, D, RW> {
   static constexpr int kChunks = D / 8;  // 16-byte chunks per head row
   // prefetch units per thread (K and V alike): (key, chunk)
   static constexpr int kUnits = kTileKeys * kChunks / 256;
+  static constexpr int kUnitKeys = 256 / kChunks;
   uint16_t k[kTileKeys * kRow];
   uint16_t v[kTileKeys * vRow];
   int last;  // the item's workgroup arrived last among its row block's partitions
@@ -816,13 +868,19 @@ __device__ __forceinline__ uint2 lds_read_tr16(const uint16_t* p) {
   const s16x4_t r = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_t*)p);
   return __builtin_bit_cast(uint2, r);
 }
+// fp32: rows D + 4 floats apart, an odd number of 16-byte chunks, so that the
+// 16 lanes of a group reading 16 bytes each of 16 K rows, or of one V row,
+// touch every bank once
 template <int D, int RW>
 struct alignas(16) TileLds<float, D, RW> {
-  static constexpr int kRow = D + 1;
-  static constexpr int vRow = D + 1;
-  static constexpr int kChunks = D / 4;        // float4 chunks per head row
-  static constexpr int kUnits = (kTileKeys * kChunks + 255) / 256;
-  static constexpr int vUnits = 0;             // V goes with K (same key, chunk)
+  static_assert(D % 16 == 0 && D <= 128, "head_dim of an fp32 tile");
+  static constexpr int kRow = D + 4;
+  static constexpr int vRow = D + 4;
+  static constexpr int kChunks = D / 4;  // 4-element chunks per head row
+  // keys a staging unit holds: the largest power of two whose chunks the 256
+  // threads hold, one each (head dims that are no power of two leave threads idle)
+  static constexpr int kUnitKeys = D > 64 ? 8 : D > 32 ? 16 : D > 16 ? 32 : 64;
+  static constexpr int kUnits = kTileKeys / kUnitKeys;
   float k[kTileKeys * kRow];
   float v[kTileKeys * vRow];
   int last;  // the item's workgroup arrived last among its row block's partitions
@@ -893,8 +951,7 @@ __device__ __forceinline__ float2 merge_partitions(const uint64_t* mlw, const ui
   };
   float M = -__builtin_inff();
   for (int p = lane; p < np; p += 64) M = fmaxf(M, lo_f(ld(mlw + p)));
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) M = fmaxf(M, __shfl_xor(M, o, 64));
+  M = wave_max_dpp(M);
   float L = 0.f, a0 = 0.f, a1 = 0.f;
   for (int p0 = 0; p0 < np; p0 += 64) {
     float wgt = 0.f;
@@ -924,88 +981,87 @@ __device__ __forceinline__ float2 merge_partitions(const uint64_t* mlw, const ui
       a0 += lo_f(x) * wt(u), a1 += hi_f(x) * wt(u);
     }
   }
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) L += __shfl_xor(L, o, 64);
+  L = wave_sum_dpp(L);
   const float inv = L > 0.f ? 1.f / L : 0.f;
   return make_float2(a0 * inv, a1 * inv);
 }
 
+// Device-scope 16-byte accesses (written through to, and read from, the point
+// of coherence of all XCDs, as the relaxed agent-scope atomics of up to 8
+// bytes are): raw buffer accesses with the device-scope cache bit. base: the
+// start of a sequence's partials, off: bytes from it (below 4 GB: the plan
+// splits at most a few hundred MB of rows).
+constexpr int kScopeDevice = 16;  // sc1
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t dev_buffer(void* base) {
+  return __builtin_amdgcn_make_buffer_rsrc(base, 0, -1, 0x00020000);
+}
+__device__ __forceinline__ f32x4_t dev_load16(__amdgpu_buffer_rsrc_t r, uint32_t off) {
+  return __builtin_bit_cast(f32x4_t, __builtin_amdgcn_raw_buffer_load_b128(r, (int)off, 0, kScopeDevice));
+}
+__device__ __forceinline__ void dev_store16(__amdgpu_buffer_rsrc_t r, uint32_t off, f32x4_t v) {
+  __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, v), r, (int)off, 0,
+                                         kScopeDevice);
+}
+
 // The merged output rows r_begin .. r_end - 1 of one (sequence, KV head)
 // row block (row r: query r / rep, head kvh rep + r % rep; the sequence's
-// first token tok0) from its np partitions' device-scope partials at
-// base: wavefront w takes rows r_begin + w, r_begin + w + kWv, ... in groups
-// of kMergeRows, lane l dims 2l and 2l + 1, with every load of a group issued
-// before the first sum (np <= kMergeFew; longer splits row by row). Groups of
-// 5 rows take a spec-verify row block (5 queries x 4 heads) in one round on 4
-// wavefronts; kernels whose item body needs fewer registers use groups of 2,
-// so that the merge does not raise their register count.
+// first token tok0) from its np partitions' device-scope partials (a row's
+// first np of `stride` partial rows; the sequence's partials start at base).
+// A wavefront takes 64 / (D / 4) rows at a time, a lane 4 dims of one of
+// them: it reads its row's (max, sum) pairs and its 16 bytes of every
+// partition, kMergeFew partitions at a time, all issued before the first use
+// (more partitions than that: an online merge over groups of them). One row
+// per wavefront at a time with 8-byte loads, and shuffles for the row's max
+// and sum, took 26 of the 55 us of one 400-query fp32 chunk (4 partitions).
 constexpr int kMergeFew = 8;
-template <typename T, int D, int kWv, int kMergeRows>
+template <typename T, int D, int kWv, int kFew = kMergeFew>
 __device__ __forceinline__ void merge_tile_rows(T* __restrict__ out, int H, int rep, int kvh,
-                                                int r_begin, int r_end, int tok0, int np,
-                                                int64_t base, const float2* ml, const float* po,
-                                                int wave, int lane) {
-  static_assert(D % 2 == 0 && D <= 128, "dim pairs per lane");
-  const bool pair_ok = 2 * lane < D;
-  const int dp = pair_ok ? lane : 0;  // lanes past the row read pair 0 and store nothing
-  auto ld = [](const uint64_t* a) {
-    return __hip_atomic_load(a, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  };
-  auto row_at = [&](int r) {  // the row's first partial row
-    const int j = r / rep;
-    return base + (int64_t)(j * H + kvh * rep + (r - j * rep)) * np;
-  };
-  auto store = [&](int r, float o0, float o1) {
-    const int j = r / rep;
-    T* dst = out + ((int64_t)(tok0 + j) * H + kvh * rep + (r - j * rep)) * D + 2 * lane;
-    if (!pair_ok) return;
-    if constexpr (sizeof(T) == 2)
-      *reinterpret_cast<uint32_t*>(dst) = cvt_pk_bf16(o0, o1);
-    else
-      *reinterpret_cast<float2*>(dst) = make_float2(o0, o1);
-  };
-  if (np > kMergeFew) {
-    for (int r = r_begin + wave; r < r_end; r += kWv) {
-      const int64_t rb = row_at(r);
-      const float2 o = merge_partitions(reinterpret_cast<const uint64_t*>(ml + rb),
-                                        reinterpret_cast<const uint64_t*>(po + rb * D) + dp, D / 2,
-                                        np, lane);
-      store(r, o.x, o.y);
-    }
-    return;
-  }
-  for (int r0 = r_begin + wave; r0 < r_end; r0 += kWv * kMergeRows) {
-    uint64_t mv[kMergeRows], xv[kMergeRows][kMergeFew];
+                                                int r_begin, int r_end, int tok0, int stride,
+                                                int np, int64_t base, const float2* ml,
+                                                const float* po, int wave, int lane) {
+  static_assert(D % 4 == 0 && D <= 128, "16-byte chunks per lane");
+  constexpr int kNC = D / 4, kRows = 64 / kNC;  // lanes per row, rows per wavefront
+  const int sub = min(lane / kNC, kRows - 1), ch = lane % kNC;
+  const __amdgpu_buffer_rsrc_t pb = dev_buffer(const_cast<float*>(po + base * D));
+  const uint64_t* mlw = reinterpret_cast<const uint64_t*>(ml + base);
+  for (int r0 = r_begin + wave * kRows; r0 < r_end; r0 += kWv * kRows) {
+    const int r = r0 + sub;
+    const int rr = min(r, r_end - 1);
+    const int j = rr / rep, head = kvh * rep + (rr - j * rep);
+    const int row = (j * H + head) * stride;  // the row's first partial row, from base
+    float M = -__builtin_inff(), L = 0.f;
+    f32x4_t a = {0.f, 0.f, 0.f, 0.f};
+    for (int p0 = 0; p0 < np; p0 += kFew) {
+      uint64_t mv[kFew];
+      f32x4_t xv[kFew];
 #pragma unroll
-    for (int g = 0; g < kMergeRows; ++g) {
-      const int64_t rb = row_at(min(r0 + kWv * g, r_end - 1));
-      mv[g] = ld(reinterpret_cast<const uint64_t*>(ml + rb) + min(lane, np - 1));
-#pragma unroll
-      for (int u = 0; u < kMergeFew; ++u)
-        xv[g][u] = ld(reinterpret_cast<const uint64_t*>(po + (rb + min(u, np - 1)) * D) + dp);
-    }
-#pragma unroll
-    for (int g = 0; g < kMergeRows; ++g) {
-      const int r = r0 + kWv * g;
-      if (r >= r_end) break;  // uniform over the wavefront
-      const float m = lo_f(mv[g]);
-      float M = lane < np ? m : -__builtin_inff();
-#pragma unroll
-      for (int o = 32; o > 0; o >>= 1) M = fmaxf(M, __shfl_xor(M, o, 64));
-      const float wgt = lane < np && m != -__builtin_inff() ? exp2_fast(m - M) : 0.f;
-      float L = lane < np ? hi_f(mv[g]) * wgt : 0.f;
-      float a0 = 0.f, a1 = 0.f;
-#pragma unroll
-      for (int u = 0; u < kMergeFew; ++u) {
-        if (u >= np) break;  // uniform
-        const float wt =
-            __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, wgt), u));
-        a0 += lo_f(xv[g][u]) * wt, a1 += hi_f(xv[g][u]) * wt;
+      for (int u = 0; u < kFew; ++u) {
+        const int p = min(p0 + u, np - 1);
+        mv[u] = __hip_atomic_load(mlw + row + p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        xv[u] = dev_load16(pb, ((uint32_t)(row + p) * D + 4 * ch) * 4);
       }
+      float Mn = M;
 #pragma unroll
-      for (int o = 32; o > 0; o >>= 1) L += __shfl_xor(L, o, 64);
-      const float inv = L > 0.f ? 1.f / L : 0.f;
-      store(r, a0 * inv, a1 * inv);
+      for (int u = 0; u < kFew; ++u) Mn = fmaxf(Mn, lo_f(mv[u]));  // repeats change nothing
+      const float alpha = M == -__builtin_inff() ? 0.f : exp2_fast(M - Mn);
+      L *= alpha, a *= alpha, M = Mn;
+#pragma unroll
+      for (int u = 0; u < kFew; ++u) {
+        if (p0 + u >= np) break;  // uniform
+        const float m = lo_f(mv[u]);
+        const float w = m != -__builtin_inff() ? exp2_fast(m - Mn) : 0.f;
+        L += hi_f(mv[u]) * w;
+        a += xv[u] * w;
+      }
+    }
+    const float inv = L > 0.f ? 1.f / L : 0.f;
+    if (r < r_end && lane < kRows * kNC) {
+      T* dst = out + ((int64_t)(tok0 + j) * H + head) * D + 4 * ch;
+      a *= inv;
+      if constexpr (sizeof(T) == 2)
+        *reinterpret_cast<uint2*>(dst) = make_uint2(cvt_pk_bf16(a[0], a[1]), cvt_pk_bf16(a[2], a[3]));
+      else
+        *reinterpret_cast<f32x4_t*>(dst) = a;
     }
   }
 }
@@ -1046,6 +1102,8 @@ __device__ __forceinline__ void tile_body(TileLds<T, D, RW>& lds, int it, int pa
   constexpr int kKS = kW ? D / 16 : kBf16 ? D / 32 : D / 4;  // k-steps of the QK^T product
   constexpr int kST = kTileKeys / (kW ? 32 : 16);        // key subtiles per LDS tile
   constexpr int kCV = kW ? 16 : 4;                       // accumulator values per subtile
+  // fp32 d tiles by the width of a V read: quads, a pair, a single one
+  constexpr int kQuads = kDT / 4, kPair = (kDT & 2) ? 1 : 0, kOdd = kDT & 1;
   using Lds = TileLds<T, D, RW>;
   using AccT = float __attribute__((ext_vector_type(kCV)));
   static_assert(!kBf16 || Lds::kUnits * 256 == kTileKeys * Lds::kChunks,
@@ -1072,8 +1130,18 @@ __device__ __forceinline__ void tile_body(TileLds<T, D, RW>& lds, int it, int pa
     // last), then from a second list in the order of item_seq (tail_seq),
     // whose offsets follow it: the last partitions
     int i, part, kvh, rb_local, q_len;
-    const bool first = !kW && it < item_off[S];
-    if (kW || !first) {
+    const bool first = kBf16 && !kW && it < item_off[S];
+    if constexpr (!kBf16) {
+      // fp32: the second list holds every partition (the first one is empty),
+      // KV heads adjacent, the later row blocks (which see more keys) first
+      const int32_t* off = item_seq + S;
+      const int pos = wave_upper_bound_le(off, S + 1, it);
+      i = item_seq[pos];
+      q_len = qsl[i + 1] - qsl[i];
+      const int local = (it - off[pos]) / Hkv, ns = nparts[i];
+      kvh = (it - off[pos]) % Hkv;
+      part = local % ns, rb_local = cdiv(q_len * rep, kItemRows) - 1 - local / ns;
+    } else if (kW || !first) {
       const int32_t* off = kW ? item_off : item_seq + S;
       const int t = kW ? it : it - item_off[S];
       const int pos = wave_upper_bound_le(off, S + 1, t);
@@ -1090,6 +1158,9 @@ __device__ __forceinline__ void tile_body(TileLds<T, D, RW>& lds, int it, int pa
     }
     const int ctx = seq_lens[i];
     const int np = kW ? 1 : nparts[i];
+    if constexpr (!kBf16) {  // a split chunk: equal parts
+      if (q_len > kSplitMaxQ) P = chunk_part_len(ctx, np);
+    }
     const int nrows = q_len * rep;
     const bool stream_kv = nrows <= kRows;  // no other pass or row block reads this K / V
     const int rb = kW ? cdiv(nrows, kItemRows) - 1 - rb_local : rb_local;
@@ -1100,6 +1171,15 @@ __device__ __forceinline__ void tile_body(TileLds<T, D, RW>& lds, int it, int pa
     // keys the block's last row can see bound the tiles the workgroup loads
     const int blk_last = min(nrows - 1, rbase + kRows - 1);
     const int kend_wg = min(kend, ctx - q_len + blk_last / rep + 1);
+    // the partitions that reach the row block's keys: of a split chunk's (fp32)
+    // row block, those past its last row's position have no work
+    int ne = np;
+    if constexpr (!kBf16) {
+      if (np > 1 && q_len > kSplitMaxQ) {
+        ne = cdiv(ctx - q_len + blk_last / rep + 1, P);
+        if (part >= ne) return;
+      }
+    }
     const int row0 = rbase + wave * RW;
     const int wave_last = min(nrows - 1, row0 + RW - 1);
     const int kend_wave = row0 < nrows ? min(kend, ctx - q_len + wave_last / rep + 1) : kbeg;
@@ -1124,7 +1204,14 @@ __device__ __forceinline__ void tile_body(TileLds<T, D, RW>& lds, int it, int pa
           uint4 w = row_ok ? *reinterpret_cast<const uint4*>(qrow + d0) : make_uint4(0, 0, 0, 0);
           qop[s] = __builtin_bit_cast(bf16x8_t, w);
         } else {
-          qop[s] = row_ok ? qrow[4 * s + grp] : 0.f;
+          // step 4 g + e of the product covers k = 16 g + 4 grp + e: a lane's
+          // operands of 4 steps are adjacent, in the query as in a K row
+          if (s % 4 == 0) {
+            const f32x4_t w = row_ok ? *reinterpret_cast<const f32x4_t*>(qrow + 4 * s + 4 * grp)
+                                     : (f32x4_t){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int e = 0; e < 4; ++e) qop[s + e] = w[e];
+          }
         }
       }
     }
@@ -1147,78 +1234,82 @@ __device__ __forceinline__ void tile_body(TileLds<T, D, RW>& lds, int it, int pa
     // 16-row bf16 items of head_dim 128 (short queries: spec-verify, HBM-bound)
     // keep three tiles' loads in flight; the others one
     constexpr bool kDeep = kBf16 && RW == 16 && D == 128;
-    uint4 pk[Lds::kUnits / kHalves], pv[Lds::kUnits / kHalves];
-    uint4 pk2[kDeep ? Lds::kUnits : 1], pv2[kDeep ? Lds::kUnits : 1];
-    uint4 pk3[kDeep ? Lds::kUnits : 1], pv3[kDeep ? Lds::kUnits : 1];
-    // bf16 staging: K unit r of a tile is keys k0 + kUnitKeys r + threadIdx / kChunks,
-    // chunk threadIdx % kChunks; with blocks of >= kUnitKeys slots the unit lies
-    // in one block whose id is uniform over the workgroup (tile starts are
-    // multiples of 64); in a head-major cache the unit is one contiguous span.
-    // Keys past the workgroup's end are masked: K reads stay in the last
-    // key's block (finite or not, the score is replaced by -inf); V reads
-    // re-read the last key, finite values whose weights are zero.
-    constexpr int kUnitKeys = 256 / Lds::kChunks;
+    // Staging: unit r of a tile is keys k0 + kUnitKeys r + tk, tk = threadIdx /
+    // kChunks, chunk threadIdx % kChunks (16 bytes of bf16; 4 elements on the
+    // fp32 path, whatever their type); with blocks of >= kUnitKeys slots the
+    // unit lies in one block whose id is uniform over the workgroup (tile
+    // starts are multiples of 64); in a head-major cache the unit is one
+    // contiguous span. Keys past the workgroup's end are masked: K reads stay
+    // in the last key's block (finite or not, the score is replaced by -inf);
+    // V reads re-read the last key, finite values whose weights are zero.
+    // Threads past the unit (fp32 head dims 48, 80, 96, 112) repeat its last
+    // key's loads and stage nothing.
+    using Raw = typename std::conditional<kBf16, uint4, typename Cache4<TKV>::Raw>::type;
+    constexpr int kU = Lds::kUnits / kHalves;  // units this thread stages
+    constexpr int kCE = kBf16 ? 8 : 4;         // elements per chunk
+    constexpr int kUnitKeys = Lds::kUnitKeys;
+    constexpr bool kIdle = kUnitKeys * Lds::kChunks < 256;  // threads past the unit
+    Raw pk[kU], pv[kU];
+    Raw pk2[kDeep ? kU : 1], pv2[kDeep ? kU : 1];
+    Raw pk3[kDeep ? kU : 1], pv3[kDeep ? kU : 1];
     const bool unit_blocks = (1 << bs_log2) >= kUnitKeys;
     const uint32_t k_thr_off =
-        (uint32_t)(tl / Lds::kChunks) * (uint32_t)slot_stride + (tl % Lds::kChunks) * 8;
+        (uint32_t)(kIdle ? min(tl / Lds::kChunks, kUnitKeys - 1) : tl / Lds::kChunks) *
+            (uint32_t)slot_stride +
+        (tl % Lds::kChunks) * kCE;
     // nt: std::true_type / std::false_type, non-temporal loads or not;
     // (pk, pv): the registers the tile lands in
-    constexpr int kU = Lds::kUnits / kHalves;  // units this thread stages
-    using Regs = uint4[kU];
+    using Regs = Raw[kU];
     auto prefetch_as = [&](int k0, auto nt, Regs& pk, Regs& pv) {
       constexpr bool kNt = decltype(nt)::value;
-      if constexpr (kBf16) {
-        if (unit_blocks) {
-          // the units' block ids first (scalar loads, issued together), then
-          // every K and V address from them; V keys past the end re-read the
-          // last key, which lies in the last unit's block, as does a unit
-          // past the end (its K reads stay there too; their scores are masked)
-          const int klast = (kend_wg - 1) & ~(kUnitKeys - 1);
-          uint32_t blk[kU];
+      if (unit_blocks) {
+        // the units' block ids first (scalar loads, issued together), then
+        // every K and V address from them; V keys past the end re-read the
+        // last key, which lies in the last unit's block, as does a unit
+        // past the end (its K reads stay there too; their scores are masked)
+        const int klast = (kend_wg - 1) & ~(kUnitKeys - 1);
+        uint32_t blk[kU];
 #pragma unroll
-          for (int r = 0; r < kU; ++r)
-            blk[r] = (uint32_t)table[min(k0 + kUnitKeys * (kHalves * r + hg), klast) >> bs_log2];
-          const int tk = tl / Lds::kChunks, tc = (tl % Lds::kChunks) * 8;
+        for (int r = 0; r < kU; ++r)
+          blk[r] = (uint32_t)table[min(k0 + kUnitKeys * (kHalves * r + hg), klast) >> bs_log2];
+        const int tk = kIdle ? min(tl / Lds::kChunks, kUnitKeys - 1) : tl / Lds::kChunks;
+        const int tc = (tl % Lds::kChunks) * kCE;
 #pragma unroll
-          for (int r = 0; r < kU; ++r) {
-            const int kr = min(k0 + kUnitKeys * (kHalves * r + hg), klast);
-            const int64_t boff = (int64_t)((uint64_t)blk[r] * blk_elems) + kv_off;
-            pk[r] = load16_kv<kNt>(kc + boff + ((uint32_t)(kr & bs_mask) * (uint32_t)slot_stride +
-                                                k_thr_off));
-            const int vkey = min(kr + tk, kend_wg - 1);
-            pv[r] = load16_kv<kNt>(vc + boff + ((uint32_t)(vkey & bs_mask) * (uint32_t)slot_stride + tc));
-          }
-        } else {
-#pragma unroll
-          for (int r = 0; r < kU; ++r) {
-            const int idx = tl + 256 * (kHalves * r + hg);
-            const int kk = idx / Lds::kChunks, cc = idx - kk * Lds::kChunks;
-            const int64_t off = row_of(min(k0 + kk, kend_wg - 1)) + cc * 8;
-            pk[r] = load16_kv<kNt>(kc + off);
-            pv[r] = load16_kv<kNt>(vc + off);
-          }
+        for (int r = 0; r < kU; ++r) {
+          const int kr = min(k0 + kUnitKeys * (kHalves * r + hg), klast);
+          const int64_t boff = (int64_t)((uint64_t)blk[r] * blk_elems) + kv_off;
+          pk[r] = load_kv<kNt, Raw>(kc + boff + ((uint32_t)(kr & bs_mask) * (uint32_t)slot_stride +
+                                                 k_thr_off));
+          const int vkey = min(kr + tk, kend_wg - 1);
+          pv[r] = load_kv<kNt, Raw>(vc + boff +
+                                    ((uint32_t)(vkey & bs_mask) * (uint32_t)slot_stride + tc));
         }
       } else {
 #pragma unroll
-        for (int r = 0; r < Lds::kUnits; ++r) {
-          const int idx = tid + 256 * r;
-          const int kk = idx / Lds::kChunks, c = idx - kk * Lds::kChunks;
-          const int key = k0 + kk;
-          const bool ok = idx < kTileKeys * Lds::kChunks && key < kend_wg;
-          const int64_t off = ok ? row_of(key) + c * 4 : 0;
-          pk[r] = ok ? load4_as_f32(kc + off) : make_uint4(0, 0, 0, 0);
-          pv[r] = ok ? load4_as_f32(vc + off) : make_uint4(0, 0, 0, 0);
+        for (int r = 0; r < kU; ++r) {
+          const int tk = kIdle ? min(tl / Lds::kChunks, kUnitKeys - 1) : tl / Lds::kChunks;
+          const int kk = kUnitKeys * (kHalves * r + hg) + tk;
+          const int64_t off = row_of(min(k0 + kk, kend_wg - 1)) + (tl % Lds::kChunks) * kCE;
+          pk[r] = load_kv<kNt, Raw>(kc + off);
+          pv[r] = load_kv<kNt, Raw>(vc + off);
         }
       }
     };
-    // one uniform branch per tile, around branch-free loads
+    // one uniform branch per tile, around branch-free loads: non-temporal
+    // (streaming) loads when no other item reads the item's K / V (a sequence
+    // whose rows fit one item: spec-verify and short chunks; measured 950 ->
+    // 870 us on the 64 x 5 verify batch), ordinary ones when the sequence's
+    // other row blocks re-read them from the cache (long prefill chunks:
+    // streaming loads there measured 281 -> 298 us)
     auto prefetch = [&](int k0, Regs& dk, Regs& dv) {
       if (stream_kv)
         prefetch_as(k0, std::true_type{}, dk, dv);
       else
         prefetch_as(k0, std::false_type{}, dk, dv);
     };
-    auto stage = [&](Lds& b, const Regs& pk, const Regs& pv) {  // registers -> LDS b
+    // registers (the tile of keys k0 ..) -> LDS b; the fp32 path stores zeros for
+    // V rows past the end, so that an infinite last V row stays one (0 x inf)
+    auto stage = [&](Lds& b, int k0, const Regs& pk, const Regs& pv) {
       if constexpr (kBf16) {
 #pragma unroll
         for (int r = 0; r < kU; ++r) {
@@ -1227,19 +1318,14 @@ __device__ __forceinline__ void tile_body(TileLds<T, D, RW>& lds, int it, int pa
           *reinterpret_cast<uint4*>(&b.k[kk * Lds::kRow + c * 8]) = pk[r];
           *reinterpret_cast<uint4*>(&b.v[kk * Lds::vRow + c * 8]) = pv[r];
         }
-      } else {
+      } else if (!kIdle || tl < kUnitKeys * Lds::kChunks) {
+        const int tk = tl / Lds::kChunks, tc = (tl % Lds::kChunks) * kCE;
 #pragma unroll
-        for (int r = 0; r < Lds::kUnits; ++r) {
-          const int idx = tid + 256 * r;
-          if (idx < kTileKeys * Lds::kChunks) {
-            const int kk = idx / Lds::kChunks, c = idx - kk * Lds::kChunks;
-            float* kd = &b.k[kk * Lds::kRow + c * 4];
-            float* vd = &b.v[kk * Lds::vRow + c * 4];
-            kd[0] = __uint_as_float(pk[r].x), kd[1] = __uint_as_float(pk[r].y);
-            kd[2] = __uint_as_float(pk[r].z), kd[3] = __uint_as_float(pk[r].w);
-            vd[0] = __uint_as_float(pv[r].x), vd[1] = __uint_as_float(pv[r].y);
-            vd[2] = __uint_as_float(pv[r].z), vd[3] = __uint_as_float(pv[r].w);
-          }
+        for (int r = 0; r < kU; ++r) {
+          const int kk = kUnitKeys * r + tk;
+          *reinterpret_cast<f32x4_t*>(&b.k[kk * Lds::kRow + tc]) = Cache4<TKV>::widen(pk[r]);
+          *reinterpret_cast<f32x4_t*>(&b.v[kk * Lds::vRow + tc]) =
+              Cache4<TKV>::widen(k0 + kk < kend_wg ? pv[r] : Raw{});
         }
       }
     };
@@ -1283,21 +1369,38 @@ __device__ __forceinline__ void tile_body(TileLds<T, D, RW>& lds, int it, int pa
         }
         __builtin_amdgcn_sched_group_barrier(0x008, kKS, 0);  // the last subtile's MFMAs
       }
+      if constexpr (!kBf16) {
+        // one 16-byte read of a K row feeds 4 steps; the subtiles' chains are
+        // independent of each other
 #pragma unroll
-      for (int t = 0; t < kST && !kW; ++t) {
+        for (int t = 0; t < kST; ++t)
+#pragma unroll
+          for (int r = 0; r < kCV; ++r) sc[t][r] = 0.f;
+#pragma unroll
+        for (int g = 0; g < D / 16; ++g) {
+          f32x4_t a[kST];
+#pragma unroll
+          for (int t = 0; t < kST; ++t)
+            a[t] = *reinterpret_cast<const f32x4_t*>(
+                &b.k[(16 * t + col) * Lds::kRow + 16 * g + 4 * grp]);
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+#pragma unroll
+            for (int t = 0; t < kST; ++t)
+              sc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[t][e], qop[4 * g + e], sc[t], 0, 0, 0);
+        }
+      }
+#pragma unroll
+      for (int t = 0; t < kST && !kW && kBf16; ++t) {
 #pragma unroll
         for (int r = 0; r < kCV; ++r) sc[t][r] = 0.f;
 #pragma unroll
         for (int s = 0; s < kKS; ++s) {
-          if constexpr (kW) {
-          } else if constexpr (kBf16) {
+          if constexpr (!kW && kBf16) {
             const uint4 w = *reinterpret_cast<const uint4*>(
                 &b.k[(16 * t + col) * Lds::kRow + 32 * s + 8 * grp]);
             sc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, w),
                                                             qop[s], sc[t], 0, 0, 0);
-          } else {
-            const float a = b.k[(16 * t + col) * Lds::kRow + 4 * s + grp];
-            sc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, qop[s], sc[t], 0, 0, 0);
           }
         }
       }
@@ -1433,16 +1536,72 @@ __device__ __forceinline__ void tile_body(TileLds<T, D, RW>& lds, int it, int pa
           }
         }
       } else {
+        // the d tiles in quads (row m of tile 4 q + e is dim 64 q + 4 m + e: one
+        // 16-byte read of a V row feeds 4 tiles), then a pair, then a single one
+        // (each key's operands are read kLookF keys before their products: left
+        // to itself the compiler reads and waits key by key)
+        constexpr int kLookF = 3;
+        float vd[kLookF][kDT];
+        auto vread_f = [&](int st, float (&vd)[kDT]) {  // key 16 (st / 4) + 4 grp + st % 4
+          const float* vrow = &b.v[(16 * (st >> 2) + 4 * grp + (st & 3)) * Lds::vRow];
 #pragma unroll
-        for (int t = 0; t < kST; ++t)
+          for (int q = 0; q < kQuads; ++q) {
+            const f32x4_t w = *reinterpret_cast<const f32x4_t*>(vrow + 64 * q + 4 * col);
 #pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            const float* vrow = &b.v[(16 * t + 4 * grp + e) * Lds::vRow];
-#pragma unroll
-            for (int u = 0; u < kDT; ++u)
-              acc[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(vrow[16 * u + col], pr[t][e], acc[u],
-                                                            0, 0, 0);
+            for (int x = 0; x < 4; ++x) vd[4 * q + x] = w[x];
           }
+          if constexpr (kPair > 0) {
+            const f32x2_t w = *reinterpret_cast<const f32x2_t*>(vrow + 64 * kQuads + 2 * col);
+            vd[4 * kQuads] = w[0], vd[4 * kQuads + 1] = w[1];
+          }
+          if constexpr (kOdd > 0) vd[kDT - 1] = vrow[16 * (kDT - 1) + col];
+        };
+        constexpr int kReads = kQuads + kPair + kOdd;  // LDS reads of a step
+#pragma unroll
+        for (int st = 0; st < kLookF; ++st) vread_f(st, vd[st]);
+#pragma unroll
+        for (int st = 0; st < 4 * kST; ++st) {
+#pragma unroll
+          for (int u = 0; u < kDT; ++u)
+            acc[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(vd[st % kLookF][u], pr[st >> 2][st & 3],
+                                                          acc[u], 0, 0, 0);
+          if (st + kLookF < 4 * kST) vread_f(st + kLookF, vd[st % kLookF]);
+        }
+        __builtin_amdgcn_sched_group_barrier(0x100, kLookF * kReads, 1);
+#pragma unroll
+        for (int st = 0; st < 4 * kST; ++st) {
+          __builtin_amdgcn_sched_group_barrier(0x008, kDT, 1);
+          if (st + kLookF < 4 * kST) __builtin_amdgcn_sched_group_barrier(0x100, kReads, 1);
+        }
+      }
+    };
+    // f(d, x0, x1, x2, x3) for every 4 adjacent dims d .. d + 3 of the lane's
+    // share of its output row
+    auto each4 = [&](auto&& f) {
+      if constexpr (kBf16) {
+#pragma unroll
+        for (int u = 0; u < kDT; ++u)
+#pragma unroll
+          for (int b4 = 0; b4 < kCV / 4; ++b4)
+            f(kW ? 32 * u + 8 * b4 + 4 * grp : 16 * u + 4 * grp, acc[u][4 * b4], acc[u][4 * b4 + 1],
+              acc[u][4 * b4 + 2], acc[u][4 * b4 + 3]);
+      } else {  // row m of a quad's, a pair's or the single d tile (see the PV product)
+#pragma unroll
+        for (int q = 0; q < kQuads; ++q)
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            f(64 * q + 4 * (4 * grp + r), acc[4 * q][r], acc[4 * q + 1][r], acc[4 * q + 2][r],
+              acc[4 * q + 3][r]);
+        if constexpr (kPair > 0) {
+          constexpr int u = 4 * kQuads;
+#pragma unroll
+          for (int r = 0; r < 4; r += 2)
+            f(64 * kQuads + 2 * (4 * grp + r), acc[u][r], acc[u + 1][r], acc[u][r + 1],
+              acc[u + 1][r + 1]);
+        }
+        if constexpr (kOdd > 0)
+          f(16 * (kDT - 1) + 4 * grp, acc[kDT - 1][0], acc[kDT - 1][1], acc[kDT - 1][2],
+            acc[kDT - 1][3]);
       }
     };
     // one tile: stage it from registers (pk, pv), refill them with the tile
@@ -1450,7 +1609,7 @@ __device__ __forceinline__ void tile_body(TileLds<T, D, RW>& lds, int it, int pa
     auto tile_step = [&](int ti, int ahead, Regs& pk, Regs& pv) {
       const int k0 = kbeg + ti * kTileKeys;
       __syncthreads();  // the previous tile (or item) is done with the LDS buffer
-      stage(lds, pk, pv);
+      stage(lds, k0, pk, pv);
       __syncthreads();
       if (ti + ahead < ntile) prefetch(k0 + ahead * kTileKeys, pk, pv);  // in flight meanwhile
       if (k0 < kend_wave) compute(lds, k0);  // else every row of the wave is past its end
@@ -1478,43 +1637,31 @@ __device__ __forceinline__ void tile_body(TileLds<T, D, RW>& lds, int it, int pa
     if constexpr (!kW) l_row += __shfl_xor(l_row, 16, 64);
     l_row += __shfl_xor(l_row, 32, 64);
     if (row_ok) {
-      if (np == 1) {
+      if (ne == 1) {
         const float inv = l_row > 0.f ? 1.f / l_row : 0.f;
         T* orow = out + ((int64_t)tok * H + head) * D;
-#pragma unroll
-        for (int u = 0; u < kDT; ++u)
-#pragma unroll
-          for (int b4 = 0; b4 < kCV / 4; ++b4) {
-            const int d = kW ? 32 * u + 8 * b4 + 4 * grp : 16 * u + 4 * grp;
-            const float x0 = acc[u][4 * b4] * inv, x1 = acc[u][4 * b4 + 1] * inv;
-            const float x2 = acc[u][4 * b4 + 2] * inv, x3 = acc[u][4 * b4 + 3] * inv;
-            if constexpr (kBf16) {
-              *reinterpret_cast<uint2*>(orow + d) = make_uint2(cvt_pk_bf16(x0, x1), cvt_pk_bf16(x2, x3));
-            } else {
-              *reinterpret_cast<float4*>(orow + d) = make_float4(x0, x1, x2, x3);
-            }
-          }
+        each4([&](int d, float x0, float x1, float x2, float x3) {
+          x0 *= inv, x1 *= inv, x2 *= inv, x3 *= inv;
+          if constexpr (kBf16)
+            *reinterpret_cast<uint2*>(orow + d) = make_uint2(cvt_pk_bf16(x0, x1), cvt_pk_bf16(x2, x3));
+          else
+            *reinterpret_cast<float4*>(orow + d) = make_float4(x0, x1, x2, x3);
+        });
       } else {
         // the partial at device scope (written through to the point of
         // coherence of all XCDs), for the row block's last workgroup
         const int64_t prow = (int64_t)split_base[i] + (int64_t)(j * H + head) * np + part;
-        uint64_t* dst = reinterpret_cast<uint64_t*>(po + prow * D);
-#pragma unroll
-        for (int u = 0; u < kDT; ++u)
-#pragma unroll
-          for (int b4 = 0; b4 < kCV / 4; ++b4) {
-            const int d = kW ? 32 * u + 8 * b4 + 4 * grp : 16 * u + 4 * grp;
-            __hip_atomic_store(dst + d / 2, pack2(acc[u][4 * b4], acc[u][4 * b4 + 1]),
-                               __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            __hip_atomic_store(dst + d / 2 + 1, pack2(acc[u][4 * b4 + 2], acc[u][4 * b4 + 3]),
-                               __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-          }
+        const __amdgpu_buffer_rsrc_t pb = dev_buffer(po + (int64_t)split_base[i] * D);
+        const uint32_t off = (uint32_t)((j * H + head) * np + part) * (D * 4);
+        each4([&](int d, float x0, float x1, float x2, float x3) {
+          dev_store16(pb, off + 4 * d, (f32x4_t){x0, x1, x2, x3});
+        });
         if (grp == 0)
           __hip_atomic_store(reinterpret_cast<uint64_t*>(ml + prow), pack2(m_run, l_row),
                              __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       }
     }
-    if (np > 1) {  // uniform over the workgroup (32-row items are never split)
+    if (ne > 1) {  // uniform over the workgroup (32-row items are never split)
       // Split rows are merged in the kernel by the last workgroup to finish a
       // partition of the row block, as the bandwidth decode kernel merges its
       // ranges: partial stores completed, then one device-scope arrival on
@@ -1528,15 +1675,15 @@ __device__ __forceinline__ void tile_body(TileLds<T, D, RW>& lds, int it, int pa
         int32_t* cnt = reinterpret_cast<int32_t*>(ml + split_base[i] + (int64_t)q_len * H * np +
                                                   kvh * nrb + rb);
         const int prev = __hip_atomic_fetch_add(cnt, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        lds.last = prev == np - 1;
-        if (prev == np - 1) __hip_atomic_store(cnt, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        lds.last = prev == ne - 1;
+        if (prev == ne - 1) __hip_atomic_store(cnt, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       }
       __syncthreads();
       if (lds.last) {
         asm volatile("" ::: "memory");  // no load below moves above the arrival
-        merge_tile_rows<T, D, kWv, kDeep ? 5 : 2>(out, H, rep, kvh, rbase,
-                                                  min(nrows, rbase + kItemRows), qsl[i], np,
-                                                  (int64_t)split_base[i], ml, po, wave, lane);
+        merge_tile_rows<T, D, kWv>(
+            out, H, rep, kvh, rbase, min(nrows, rbase + kItemRows), qsl[i], np, ne,
+            (int64_t)split_base[i], ml, po, wave, lane);
       }
     }
   }
@@ -1581,7 +1728,8 @@ __device__ __forceinline__ int claimed_item(int64_t c, int stride, int base, int
 // zeroed by the plan and, at the end of every run, by the claims that return
 // each queue's last value (below).
 template <typename T, int D, int RW, int kWv, typename TKV = T>
-__global__ void __launch_bounds__(64 * kWv) __attribute__((amdgpu_waves_per_eu(2))) attend_tile_kernel(
+__global__ void __launch_bounds__(64 * kWv)
+__attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 && D <= 64 ? 3 : 2))) attend_tile_kernel(
     VL_ATTN_PARAMS_KV(T, TKV), const int32_t* __restrict__ hdr, const int32_t* __restrict__ item_off,
     const int32_t* __restrict__ item_seq, int32_t* counters) {
   __shared__ TileLds<T, D, RW> lds;
@@ -1611,7 +1759,9 @@ __global__ void __launch_bounds__(64 * kWv) __attribute__((amdgpu_waves_per_eu(2
     __syncthreads();  // the item is done with the LDS; claim_lds has been read
     if (threadIdx.x == 0) claim_lds = nxt;
     __syncthreads();
-    it = claim_lds;
+    // one value for the whole workgroup, and known to be: what follows from it
+    // (sequence, partition, block ids) stays in scalar registers and loads
+    it = __builtin_amdgcn_readfirstlane(claim_lds);
   }
 }
 
@@ -2643,10 +2793,12 @@ int do_plan(const Args& a, void* ws, size_t ws_bytes, hipStream_t st) {
   // a few bandwidth-kernel items per resident workgroup
   const int target_items = fast ? kItemsPerWg * decode_grid() : 0;
   const int tile_target = kTileItemsPerWg * tile_grid();
+  const int chunk_target = kChunkItemsPerCu * vl_num_cus();
   const bool wide = tile && a.dtype == VL_DTYPE_BF16;
   auto* plan = a.S <= kPlanThreads * kPlanRegSeqs ? plan_kernel<true> : plan_kernel<false>;
   plan<<<1, kPlanThreads, 0, st>>>(a.seq_lens, a.qsl, a.S, a.H, a.Hkv, fast, tile, wide,
-                                   L.cap_rows, target_items, tile_target, L.hdr, L.gen_off,
+                                   L.cap_rows, target_items, tile_target, chunk_target,
+                                   L.hdr, L.gen_off,
                                    L.tile_off, L.nparts, L.split_base, L.wide_off, L.cmb_seq,
                                    L.wide_seq, L.tail_seq, L.tail_off, L.desc, L.ml);
   VL_CHECK_LAUNCH();
@@ -2879,7 +3031,14 @@ extern "C" size_t vl_paged_attention_workspace_size(int num_seqs, int num_tokens
       std::min<int64_t>(S * H * cdiv64(ctx, 64),
                         4 * kItemsPerWg * (int64_t)decode_grid() +
                             S * H * (cdiv64(ctx, kRangeMax) + 1));
-  const int64_t rows = std::max(rows_tile, rows_fast);
+  // split fp32 chunks: sum q H np <= 2 sum q H c / P2 (np >= 2 parts), with P2
+  // >= sum c nrb Hkv / (items aimed for) and q H <= kTileRows nrb Hkv; twice
+  // that covers the arrival counters and rounding
+  const int64_t rows_chunk =
+      ctx > kChunkPart ? std::min<int64_t>(4ll * kTileRows * kChunkItemsPerCu * vl_num_cus(),
+                                           2 * num_tokens * H * (cdiv64(ctx, kChunkPart) + 1))
+                       : 0;
+  const int64_t rows = std::max(rows_tile + rows_chunk, rows_fast);
   return fixed_bytes(num_seqs) + (size_t)rows * row_bytes(head_dim);
 }
 
