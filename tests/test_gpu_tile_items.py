@@ -47,3 +47,59 @@ def test_fp32_chunk_parts_leave_their_counters_clear():
         out = torch.empty_like(q)
         o.paged_attention_run(out, q, kc, vc, bt, sl, qsl, b["scale"], 16, ws, max_query_len=200)
         check(to_np(out), oracle_attention(b), "f32")
+
+
+# every head dim whose tiles came with no alignment rule: idle staging threads
+# (80, 96, 112: units of 8 keys on 160 .. 224 threads), d tiles as quads +
+# single, quads + pair, quads + pair + single; bf16 16 / 32 / 48 widened
+@pytest.mark.parametrize("dtype,D", [("bf16", 16), ("bf16", 32), ("bf16", 48), ("bf16", 80),
+                                     ("bf16", 96), ("bf16", 112), ("f32", 80), ("f32", 96),
+                                     ("f32", 112)])
+@pytest.mark.parametrize("bs", [4, 16, 32])
+@pytest.mark.parametrize("layout", ["token", "head"])
+def test_widened_head_dims(dtype, D, bs, layout):
+    seqs = [(37, 37), (1, 2000), (70, 133), (1, 1), (5, 700), (0, 9), (17, 500)]
+    b = make_batch(seqs, 6, 3, D, bs, seed=D + bs)
+    check(run_attention(b, dtype, layout=layout), expected(b, dtype), dtype)
+
+
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+def test_widened_head_dim_takes_any_alignment(dtype):
+    """Query rows, outputs and caches at odd element offsets and strides."""
+    o = ops()
+    tdt = torch.float32 if dtype == "f32" else torch.bfloat16
+    b = make_batch([(40, 90), (1, 700), (3, 3)], 4, 2, 80, 16, seed=9)
+    S, T = len(b["seq_lens"]), b["q"].shape[0]
+
+    def odd(x):  # a contiguous copy one element into its storage
+        t = dev(x, tdt)
+        flat = torch.empty(t.numel() + 1, dtype=tdt, device="cuda")
+        v = flat[1:].view(t.shape)
+        v.copy_(t)
+        return v
+
+    wide = torch.zeros(T, 4 * 80 + 3, dtype=tdt, device="cuda")
+    q = wide[:, 1:1 + 320].view(T, 4, 80) if T == 1 else wide[:, 1:321].unflatten(1, (4, 80))
+    q.copy_(dev(b["q"], tdt))
+    out = odd(np.zeros_like(b["q"]))
+    ws = o.AttentionWorkspace().get(o.paged_attention_workspace_size(S, T, 4, 80, 700))
+    o.paged_attention(out, q, odd(b["k_cache"]), odd(b["v_cache"]), dev(b["block_tables"]),
+                      dev(b["seq_lens"]), dev(b["qsl"]), b["scale"], 16, ws, max_query_len=40)
+    check(to_np(out), expected(b, dtype), dtype)
+
+
+@pytest.mark.parametrize("D", [80, 112])
+def test_widened_head_dims_over_an_fp8_cache(D):
+    from oracle.attention import fp8_e4m3_decode, fp8_e4m3_encode
+    o = ops()
+    b = make_batch([(30, 300), (1, 900), (2, 2)], 4, 2, D, 16, seed=D)
+    enc = {n: fp8_e4m3_encode(b[n]) for n in ("k_cache", "v_cache")}
+    kc, vc = (dev(enc[n]).view(torch.float8_e4m3fn) for n in ("k_cache", "v_cache"))
+    q = dev(b["q"])
+    out = torch.empty_like(q)
+    ws = o.AttentionWorkspace().get(o.paged_attention_workspace_size(3, 33, 4, D, 900))
+    o.paged_attention(out, q, kc, vc, dev(b["block_tables"]), dev(b["seq_lens"]), dev(b["qsl"]),
+                      b["scale"], 16, ws, max_query_len=30)
+    want = oracle_attention(dict(b, k_cache=fp8_e4m3_decode(enc["k_cache"]),
+                                 v_cache=fp8_e4m3_decode(enc["v_cache"])))
+    check(to_np(out), want, "f32")

@@ -18,10 +18,12 @@
 //           per-KV-head / block-16 shape go to the bandwidth kernel (a
 //           workgroup per (range, KV head) item, its 4 wavefronts splitting
 //           the range's blocks), which merges its own split sequences;
-//           multi-query sequences go to the MFMA tile kernels (16- or 32-row
-//           wavefronts) when the head dim has an instantiation, else to the
-//           generic kernel (one wavefront per (sequence, query, head,
-//           partition)); a batch holding both kinds runs in the one step
+//           multi-query sequences, and every sequence of the other shapes, go
+//           to the MFMA tile kernels (16- or 32-row wavefronts) when the head
+//           dim is a multiple of 16 up to 128 and the block size a power of
+//           two, else to the generic kernel (one wavefront per (sequence,
+//           query, head, partition): 24 decodes + 2 chunks at head_dim 80
+//           took 784 us there, 66 on widened fp32 tiles); a batch holding both kinds runs in the one step
 //           kernel. Split sequences are merged (max-rescaled log-sum-exp)
 //           by the last workgroup to finish a partition of them, in the
 //           bandwidth, tile and step kernels, and by the combine kernel
@@ -55,7 +57,8 @@ constexpr int kHdrInts = 64;  // [0] bandwidth-kernel items [1] generic items [2
 constexpr int kPlanThreads = 256;
 constexpr int kMaxHeadDim = 256;
 constexpr int kSplitMaxQ = 16;  // only sequences with <= this many queries split their context
-constexpr int kPart0 = 64;  // first partition length tried by the planner
+constexpr int kPart0Log2 = 6;
+constexpr int kPart0 = 1 << kPart0Log2;  // first partition length tried by the planner
 // fp32 tile items of longer query chunks are cut over the context too, into
 // about this many items per compute unit, but not below kChunkPart keys each
 constexpr int kChunkItemsPerCu = 3;
@@ -65,7 +68,8 @@ constexpr float kLog2e = 1.4426950408889634f;
 // bandwidth-kernel shape
 constexpr int kFD = 128;   // head_dim
 constexpr int kFRep = 4;   // query heads per KV head
-constexpr int kFBs = 16;   // block size
+constexpr int kFBsLog2 = 4;
+constexpr int kFBs = 1 << kFBsLog2;  // block size
 constexpr int kFChunk = 16;  // blocks per softmax chunk (256 tokens)
 constexpr int kBK = 4;  // blocks per K load burst (decode kernel)
 constexpr int kBV = 2;  // blocks per V load burst (decode kernel)
@@ -154,12 +158,23 @@ inline bool fast_shape(int dtype, int H, int Hkv, int D, int bs) {
   return dtype == VL_DTYPE_BF16 && D == kFD && bs == kFBs && Hkv % 4 == 0 && H == kFRep * Hkv;
 }
 
-// head_dims with an MFMA tile instantiation
+// head_dims with an MFMA tile instantiation: every multiple of 16 up to 128
 inline bool tile_shape(int dtype, int D, int bs) {
   if (bs <= 0 || (bs & (bs - 1)) != 0) return false;  // block math is shifts and masks
-  if (dtype == VL_DTYPE_BF16) return D == 64 || D == 128;
-  // fp32, and fp32 queries over bf16 / FP8 E4M3 caches (widened when staged)
-  return D == 16 || D == 32 || D == 48 || D == 64 || D == 128;
+  return D > 0 && D % 16 == 0 && D <= 128;
+}
+
+// bf16 head dims whose products run on bf16 operands (the weights rounded to
+// bf16); the others widen bf16 to fp32 and run as fp32, weights included
+inline bool bf16_tile_shape(int dtype, int D) {
+  return dtype == VL_DTYPE_BF16 && (D == 64 || D == 128);
+}
+
+// Tile shapes whose operands must be 16-byte aligned (query rows a multiple
+// of 8 elements); the other head dims take any alignment, by accesses the
+// compiler is told may be unaligned (the same instructions on gfx950)
+constexpr bool aligned_tile_dim(bool bf16, int D) {
+  return D == 64 || D == 128 || (!bf16 && (D == 16 || D == 32 || D == 48));
 }
 
 __device__ __forceinline__ int upper_bound_le(const int32_t* a, int n, int x) {
@@ -270,44 +285,64 @@ struct SeqWork {
 // generic kernel.
 __device__ __forceinline__ bool is_bw(int q, int c, bool fast) { return fast && q == 1 && c > 0; }
 
-// P2 > 0: fp32 tile chunks (q > kSplitMaxQ) are split too, into equal parts
-// of about P2 keys (whole key tiles; the tile kernel derives the length from
-// the part count, chunk_part_len).
+// P and R are powers of two, kept as their logarithms: an integer division is
+// ~30 instructions, and a plan of a few sequences is a chain of such steps.
+struct PlanLens {
+  int lp;  // short queries: log2 of the partition length P
+  int p2;  // fp32 tile chunks (q > kSplitMaxQ): keys per part aimed for, or kNoSplit
+  int lr;  // decode ranges: log2 of R
+};
+constexpr int kNoSplit = 1 << 30;
+constexpr int kMaxLen = 29;  // log2 of the longest length tried
+
+// Keys per part of a chunk of context c cut into np parts: equal parts of
+// whole key tiles (a power of two with a short rest measured 113 against 101
+// us for 24 decodes + 5 chunks, 152 against 114 for 10 chunks). The tile
+// kernel derives the length from the part count with the same formula.
 __device__ __forceinline__ int chunk_part_len(int c, int np) {
   return cdiv(cdiv(c, kTileKeys), np) * kTileKeys;
 }
 
-__device__ __forceinline__ SeqWork seq_work(int q, int c, int P, int P2, int R, int H, int Hkv,
+__device__ __forceinline__ int cdiv_pow2(int a, int l) { return (int)(((int64_t)a + (1 << l) - 1) >> l); }
+
+__device__ __forceinline__ SeqWork seq_work(int q, int c, const PlanLens& n, int rep, int Hkv,
                                             bool fast, bool tile, bool wide) {
   SeqWork w;
   const bool live = q > 0 && c > 0;
   const bool bw = is_bw(q, c, fast);
   const bool tl = !bw && tile && live;
   if (bw) {
-    w.np = (c + R - 1) / R;
-    w.full = c / R;
-    w.tail = (c % R) != 0;
+    w.np = cdiv_pow2(c, n.lr);
+    w.full = c >> n.lr;
+    w.tail = (c & ((1 << n.lr) - 1)) != 0;
   } else {
-    w.np = (q > 0 && q <= kSplitMaxQ && c > P) ? (c + P - 1) / P : 1;
-    if (tl && !wide && q > kSplitMaxQ && P2 > 0 && c > P2)
-      w.np = cdiv(c, chunk_part_len(c, cdiv(c, P2)));  // no part is empty
+    w.np = q > 0 && q <= kSplitMaxQ && c > 0 ? cdiv_pow2(c, n.lp) : 1;
+    if (tl && !wide && q > kSplitMaxQ && c > n.p2)
+      w.np = cdiv(c, chunk_part_len(c, cdiv(c, n.p2)));  // no part is empty
     w.full = w.tail = 0;
   }
   const bool wd = tl && wide && q > kSplitMaxQ;  // never split (np == 1)
-  w.tile = tl && !wd ? (int64_t)w.np * Hkv * cdiv(q * (H / Hkv), kTileRows) : 0;
-  w.wide = wd ? (int64_t)Hkv * cdiv(q * (H / Hkv), kWideRows) : 0;
-  w.gen = (bw || tl) ? 0 : (int64_t)max(q, 0) * H * w.np;
+  const int64_t blocks = tl && !wd ? (int64_t)Hkv * cdiv(q * rep, kTileRows) : 0;
+  w.tile = w.np * blocks;
+  w.wide = wd ? (int64_t)Hkv * cdiv(q * rep, kWideRows) : 0;
+  w.gen = (bw || tl) ? 0 : (int64_t)max(q, 0) * rep * Hkv * w.np;
   // a split decode sequence also keeps one arrival counter per KV head in
   // the rows after its partials, a split 16-row tile sequence one per (KV
   // head, row block)
-  w.rows = w.np > 1 ? (int64_t)q * H * w.np + (bw ? Hkv : w.tile > 0 ? w.tile / w.np : 0) : 0;
+  w.rows = w.np > 1 ? (int64_t)q * rep * Hkv * w.np + (bw ? Hkv : blocks) : 0;
   return w;
 }
 
-constexpr int kRangeMax = 2048;       // longest decode range the planner starts with
+constexpr int kRangeMaxLog2 = 11;
+constexpr int kRangeMax = 1 << kRangeMaxLog2;  // longest decode range the planner starts with
 constexpr int kItemsPerWg = 4;  // decode items aimed for per resident workgroup
 constexpr int kTileItemsPerWg = 4;  // split tile items aimed for per workgroup
-constexpr int kTailBuckets = 1024;
+// fp32 ones have more work per key and pay their start and merge more often:
+// 24 decodes at head_dim 80 68 us at 4, 54 at 2, 48 at 1, with 2 chunks beside
+// them 79, 66 and 76
+constexpr int kTileItemsPerWgF32 = 2;
+constexpr int kTailBucketsLog2 = 10;
+constexpr int kTailBuckets = 1 << kTailBucketsLog2;
 constexpr int kPlanLdsSeqs = 2048;  // batches the plan keeps per-sequence counts of in LDS
 constexpr int kPlanBuckets = kTailBuckets / kPlanThreads;  // buckets owned by each plan thread
 constexpr int kPlanRegSeqs = 4;  // sequences a plan thread keeps in registers (S <= 1024)
@@ -423,7 +458,7 @@ __device__ __forceinline__ int bucket_add(int* h, int key, int hot) {
 // histogram; sums are wavefront reductions, not same-address atomics.
 template <bool kCached>
 __global__ void __launch_bounds__(kPlanThreads) plan_kernel(
-    const int32_t* __restrict__ seq_lens, const int32_t* __restrict__ qsl, int S, int H, int Hkv,
+    const int32_t* __restrict__ seq_lens, const int32_t* __restrict__ qsl, int S, int rep, int Hkv,
     bool fast, bool tile, bool wide, int64_t cap_rows, int target_items, int tile_target,
     int chunk_target, int32_t* __restrict__ hdr, int32_t* __restrict__ gen_off,
     int32_t* __restrict__ tile_off, int32_t* __restrict__ nparts,
@@ -446,28 +481,38 @@ __global__ void __launch_bounds__(kPlanThreads) plan_kernel(
   // 0. range length from the decode tokens and the target item count; the
   // same for the partition length of the splittable multi-query sequences
   // (at most kSplitMaxQ queries), counted in (KV head, 64-row block) units
-  int R = 64, P = kPart0, P2 = 0;
+  PlanLens n = {kPart0Log2, kNoSplit, 6};
   bool lpt;  // 16-row items (or bf16 ones' last partitions) handed out longest first
   {
-    const int rep = H / Hkv;
     unsigned long long v[3] = {0, 0, 0};
     ch.each(qsl, seq_lens, [&](int, int q, int c) {
-      if (is_bw(q, c, fast))
+      if (is_bw(q, c, fast)) {
         v[0] += (unsigned long long)c;
-      else if (tile && q > 0 && c > 0)
-        v[q <= kSplitMaxQ ? 1 : 2] += (unsigned long long)c * cdiv(q * rep, kTileRows);
+      } else if (tile && q > 0 && c > 0) {
+        const unsigned long long u = (unsigned long long)c * cdiv(q * rep, kTileRows);
+        v[1] += q <= kSplitMaxQ ? u : 0;
+        v[2] += q <= kSplitMaxQ ? 0 : u;
+      }
     });
-    plan_sum(v, red0);  // its barrier also orders the histogram clearing
-    while (R < kRangeMax && v[0] * (unsigned long long)Hkv >
-                                (unsigned long long)max(target_items, 1) * (unsigned long long)R)
-      R *= 2;
-    while (P < (1 << 20) && v[1] * (unsigned long long)Hkv >
-                                (unsigned long long)max(tile_target, 1) * (unsigned long long)P)
-      P *= 2;
-    if (tile && !wide && v[2] > 0) {
-      const unsigned long long len = v[2] * (unsigned long long)Hkv / max(chunk_target, 1);
-      P2 = (int)min((unsigned long long)(1 << 29), max((unsigned long long)kChunkPart, len));
-    }
+    if (tile && !wide) {
+      plan_sum<3>(v, red0);
+    } else {  // nobody cuts longer queries over the context
+      unsigned long long v2[2] = {v[0], v[1]};
+      plan_sum<2>(v2, reinterpret_cast<unsigned long long(*)[2]>(red0));
+      v[0] = v2[0], v[1] = v2[1], v[2] = 0;
+    }  // (the sum's barrier also orders the histogram clearing)
+    // the smallest length, at least `from`, that leaves at most `target` items
+    auto fit = [&](unsigned long long keys, int target, int from, int to) {
+      int l = from;
+      while (l < to && keys * (unsigned long long)Hkv > (unsigned long long)max(target, 1) << l) ++l;
+      return l;
+    };
+    n.lr = fit(v[0], target_items, 6, kRangeMaxLog2);
+    n.lp = fit(v[1], tile_target, kPart0Log2, 20);
+    if (v[2] > 0)
+      n.p2 = (int)min((unsigned long long)kNoSplit,
+                      max((unsigned long long)kChunkPart,
+                          v[2] * (unsigned long long)Hkv / max(chunk_target, 1)));
     lpt = wide ? v[1] > 0 : v[1] + v[2] > 0;
   }
   // 1. double P and R until the split partials fit (every thread holds the
@@ -475,23 +520,22 @@ __global__ void __launch_bounds__(kPlanThreads) plan_kernel(
   for (int it = 0;; ++it) {
     unsigned long long need[1] = {0};
     ch.each(qsl, seq_lens, [&](int, int q, int c) {
-      need[0] += seq_work(q, c, P, P2, R, H, Hkv, fast, tile, wide).rows;
+      need[0] += seq_work(q, c, n, rep, Hkv, fast, tile, wide).rows;
     });
     plan_sum(need, red1[it & 1]);
-    if (need[0] <= (unsigned long long)cap_rows || (P >= (1 << 29) && R >= (1 << 29))) break;
-    if (P2 > 0)
-      P2 = 0;  // the chunks' partials do not fit beside the others: leave them whole
+    if (need[0] <= (unsigned long long)cap_rows || (n.lp >= kMaxLen && n.lr >= kMaxLen)) break;
+    if (n.p2 != kNoSplit)
+      n.p2 = kNoSplit;  // the chunks' partials do not fit beside the others: leave them whole
     else
-      P = min(P * 2, 1 << 29), R = min(R * 2, 1 << 29);
+      n.lp = min(n.lp + 1, kMaxLen), n.lr = min(n.lr + 1, kMaxLen);
   }
+  const int R = 1 << n.lr, P = 1 << n.lp;
   // 2. offsets
   // tail ranges are bucketed by their length in blocks, longest first
-  const int rblocks = R / kFBs;
+  const int rshift = max(0, n.lr - kFBsLog2 - kTailBucketsLog2);  // of more blocks than buckets
   auto tail_key = [&](int c) {
-    const int blocks = ((c % R) + kFBs - 1) / kFBs;  // 1 .. rblocks
-    const int k = rblocks <= kTailBuckets ? blocks - 1
-                                          : (int)((int64_t)(blocks - 1) * kTailBuckets / rblocks);
-    return kTailBuckets - 1 - k;  // ascending key = descending length
+    const int blocks = ((c & (R - 1)) + kFBs - 1) / kFBs;  // 1 .. R / kFBs
+    return kTailBuckets - 1 - ((blocks - 1) >> rshift);  // ascending key = descending length
   };
   // sequences with 32-row items by their context in 64-key tiles (up to
   // kTailBuckets - 2 distinct lengths), descending; the others in the last bucket
@@ -509,18 +553,21 @@ __global__ void __launch_bounds__(kPlanThreads) plan_kernel(
   // (32 fp32 MFMA cycles per 16 x 16 x 4 product) with one-tile decode items,
   // and the chunk items have to start first.
   auto split_items = [&](const SeqWork& w) -> int64_t {
-    return !lpt ? w.tile : w.tile > 0 && wide ? w.tile / w.np * (w.np - 1) : 0;
+    if (!lpt) return w.tile;
+    // (np is 1 for most: no division there)
+    return wide && w.np > 1 ? w.tile / w.np * (w.np - 1) : 0;
   };
   auto last_key = [&](int q, int c, const SeqWork& w) {
     if (w.tile == 0 || !lpt) return kTailBuckets - 1;
     const int64_t last = wide ? (int64_t)c - (int64_t)(w.np - 1) * P  // 1 .. P keys (all of c unsplit)
-                         : q > kSplitMaxQ ? chunk_part_len(c, w.np)
-                                          : min(c, P);
+                         : q > kSplitMaxQ && w.np > 1 ? chunk_part_len(c, w.np)
+                         : q > kSplitMaxQ             ? c
+                                                      : min(c, P);
     return kTailBuckets - 2 - (int)min<int64_t>(kTailBuckets - 2, cdiv64(last, kTileKeys) - 1);
   };
   int64_t f = 0, g = 0, r = 0, x = 0, xs = 0, tl = 0, wd = 0, cm = 0;
   ch.each(qsl, seq_lens, [&](int, int q, int c) {
-    const SeqWork w = seq_work(q, c, P, P2, R, H, Hkv, fast, tile, wide);
+    const SeqWork w = seq_work(q, c, n, rep, Hkv, fast, tile, wide);
     f += w.full, g += w.gen, r += w.rows, x += w.tile, tl += w.tail, wd += w.wide;
     xs += split_items(w);
     cm += w.np > 1 && w.gen > 0;  // the combine kernel merges only the generic kernel's splits
@@ -557,7 +604,7 @@ __global__ void __launch_bounds__(kPlanThreads) plan_kernel(
   }
   __syncthreads();
   ch.each(qsl, seq_lens, [&](int i, int q, int c) {
-    const SeqWork w = seq_work(q, c, P, P2, R, H, Hkv, fast, tile, wide);
+    const SeqWork w = seq_work(q, c, n, rep, Hkv, fast, tile, wide);
     const int qs = qsl[i];
     for (int k = 0; k < w.full; ++k) desc[fo + k] = make_int4(i, k, c, qs);
     gen_off[i] = (int32_t)go;
@@ -577,11 +624,11 @@ __global__ void __launch_bounds__(kPlanThreads) plan_kernel(
     if (w.tail) {
       const int key = tail_key(c);
       desc[tf + bucket_add<true>(hist, key, __builtin_amdgcn_readfirstlane(key))] =
-          make_int4(i, c / R, c, qs);
+          make_int4(i, c >> n.lr, c, qs);
     }
     if (w.np > 1 && w.gen > 0) cmb_seq[co++] = i;
     if (w.np > 1 && w.gen == 0)  // arrival counters start at 0
-      for (int64_t k = (int64_t)q * H * w.np; k < w.rows; ++k)
+      for (int64_t k = (int64_t)q * rep * Hkv * w.np; k < w.rows; ++k)
         reinterpret_cast<int32_t*>(ml + ro + k)[0] = 0;
     fo += w.full, go += w.gen, ro += w.rows, xo += split_items(w);
   });
@@ -594,12 +641,12 @@ __global__ void __launch_bounds__(kPlanThreads) plan_kernel(
     auto wide_items = [&](int p) -> int64_t {
       if (S <= kPlanLdsSeqs) return wcnt[p];
       const int i = wide_seq[p];
-      return seq_work(qsl[i + 1] - qsl[i], seq_lens[i], P, P2, R, H, Hkv, fast, tile, wide).wide;
+      return seq_work(qsl[i + 1] - qsl[i], seq_lens[i], n, rep, Hkv, fast, tile, wide).wide;
     };
     auto last_items = [&](int p) -> int64_t {
       if (S <= kPlanLdsSeqs) return tcnt[p];
       const int i = tail_seq[p];
-      const SeqWork w = seq_work(qsl[i + 1] - qsl[i], seq_lens[i], P, P2, R, H, Hkv, fast, tile, wide);
+      const SeqWork w = seq_work(qsl[i + 1] - qsl[i], seq_lens[i], n, rep, Hkv, fast, tile, wide);
       return w.tile - split_items(w);
     };
     int64_t mw = 0, mt = 0;
@@ -820,12 +867,55 @@ struct Cache4<uint8_t> {
   }
 };
 
+// Two floats to packed bf16 with the hardware conversion (v_cvt_pk_bf16_f32,
+// round to nearest even, as f32_to_bf16 for every finite value).
+__device__ __forceinline__ uint32_t cvt_pk_bf16(float lo, float hi) {
+  const bf16x2_t v = {(__bf16)lo, (__bf16)hi};
+  return __builtin_bit_cast(uint32_t, v);
+}
+
+// A vector type at any address.
+template <typename Raw>
+struct Loose {
+  typedef Raw T __attribute__((aligned(1)));
+};
+
+// 4 query elements as floats, and 4 output elements stored, at a row's dims
+// d .. d + 3 (kLoose: at any alignment).
+template <bool kLoose>
+__device__ __forceinline__ f32x4_t load4(const float* p) {
+  if constexpr (kLoose) return *reinterpret_cast<const typename Loose<f32x4_t>::T*>(p);
+  return *reinterpret_cast<const f32x4_t*>(p);
+}
+template <bool kLoose>
+__device__ __forceinline__ f32x4_t load4(const uint16_t* p) {
+  if constexpr (kLoose)
+    return Cache4<uint16_t>::widen(*reinterpret_cast<const typename Loose<u32x2_t>::T*>(p));
+  return Cache4<uint16_t>::widen(*reinterpret_cast<const u32x2_t*>(p));
+}
+template <bool kLoose>
+__device__ __forceinline__ void store4(float* p, f32x4_t v) {
+  if constexpr (kLoose)
+    *reinterpret_cast<typename Loose<f32x4_t>::T*>(p) = v;
+  else
+    *reinterpret_cast<f32x4_t*>(p) = v;
+}
+template <bool kLoose>
+__device__ __forceinline__ void store4(uint16_t* p, f32x4_t v) {
+  const u32x2_t w = {cvt_pk_bf16(v[0], v[1]), cvt_pk_bf16(v[2], v[3])};
+  if constexpr (kLoose)
+    *reinterpret_cast<typename Loose<u32x2_t>::T*>(p) = w;
+  else
+    *reinterpret_cast<u32x2_t*>(p) = w;
+}
+
 // K / V cache bytes of a tile item (a Raw of them), by a non-temporal
 // (streaming) load or not. The choice is a compile-time one: a runtime one
 // puts every load in a branch of its own, and the compiler then cannot issue
 // a tile's loads (and the block-id loads they need) together.
-template <bool kStream, typename Raw>
+template <bool kStream, typename Raw, bool kLoose = false>
 __device__ __forceinline__ Raw load_kv(const void* p) {
+  if constexpr (kLoose) return *reinterpret_cast<const typename Loose<Raw>::T*>(p);
   if constexpr (std::is_same<Raw, uint4>::value) {
     if constexpr (kStream)
       return __builtin_bit_cast(uint4,
@@ -891,13 +981,6 @@ __device__ __forceinline__ uint32_t pack_bf16x2(float lo, float hi) {
 }
 
 
-
-// Two floats to packed bf16 with the hardware conversion (v_cvt_pk_bf16_f32,
-// round to nearest even, as f32_to_bf16 for every finite value).
-__device__ __forceinline__ uint32_t cvt_pk_bf16(float lo, float hi) {
-  const bf16x2_t v = {(__bf16)lo, (__bf16)hi};
-  return __builtin_bit_cast(uint32_t, v);
-}
 
 // threadIdx.x, with kOpaque through an opaque move: values an item derives
 // from it are then recomputed per item instead of being hoisted out of a
@@ -1014,7 +1097,7 @@ __device__ __forceinline__ void dev_store16(__amdgpu_buffer_rsrc_t r, uint32_t o
 // per wavefront at a time with 8-byte loads, and shuffles for the row's max
 // and sum, took 26 of the 55 us of one 400-query fp32 chunk (4 partitions).
 constexpr int kMergeFew = 8;
-template <typename T, int D, int kWv, int kFew = kMergeFew>
+template <typename T, int D, int kWv, bool kLoose = false, int kFew = kMergeFew>
 __device__ __forceinline__ void merge_tile_rows(T* __restrict__ out, int H, int rep, int kvh,
                                                 int r_begin, int r_end, int tok0, int stride,
                                                 int np, int64_t base, const float2* ml,
@@ -1058,10 +1141,7 @@ __device__ __forceinline__ void merge_tile_rows(T* __restrict__ out, int H, int 
     if (r < r_end && lane < kRows * kNC) {
       T* dst = out + ((int64_t)(tok0 + j) * H + head) * D + 4 * ch;
       a *= inv;
-      if constexpr (sizeof(T) == 2)
-        *reinterpret_cast<uint2*>(dst) = make_uint2(cvt_pk_bf16(a[0], a[1]), cvt_pk_bf16(a[2], a[3]));
-      else
-        *reinterpret_cast<f32x4_t*>(dst) = a;
+      store4<kLoose>(dst, a);
     }
   }
 }
@@ -1077,11 +1157,11 @@ __device__ __forceinline__ void merge_tile_rows(T* __restrict__ out, int H, int 
 // kernel's 4; each K/V tile read from LDS feeds twice the rows). With RW 32
 // a lane holds row l%32; its S^T values are keys 32t + 8(r/4) + 4(l/32) + r%4
 // (r < 16) and its O^T values dims 32u + 8(r/4) + 4(l/32) + r%4.
-template <typename T, int D, int RW, bool kMixed, int kWv = 4, typename TKV = T>
+template <typename T, int D, int RW, bool kMixed, int kWv = 4, typename TKV = T, typename TIO = T>
 __device__ __forceinline__ void tile_body(TileLds<T, D, RW>& lds, int it, int pass, int P,
                                           const int32_t* __restrict__ item_off,
                                           const int32_t* __restrict__ item_seq,
-                                          VL_ATTN_PARAMS_KV(T, TKV)) {
+                                          VL_ATTN_PARAMS_KV(TIO, TKV)) {
   const int tid = item_tid<kMixed>();
   constexpr bool kBf16 = sizeof(T) == 2;
   constexpr bool kW = RW == 32;
@@ -1104,6 +1184,9 @@ __device__ __forceinline__ void tile_body(TileLds<T, D, RW>& lds, int it, int pa
   constexpr int kCV = kW ? 16 : 4;                       // accumulator values per subtile
   // fp32 d tiles by the width of a V read: quads, a pair, a single one
   constexpr int kQuads = kDT / 4, kPair = (kDT & 2) ? 1 : 0, kOdd = kDT & 1;
+  // head dims without an alignment rule
+  constexpr bool kLoose = !kBf16 && !aligned_tile_dim(sizeof(TIO) == 2, D);
+  static_assert(!kBf16 || std::is_same<T, TIO>::value, "bf16 tiles read and write bf16");
   using Lds = TileLds<T, D, RW>;
   using AccT = float __attribute__((ext_vector_type(kCV)));
   static_assert(!kBf16 || Lds::kUnits * 256 == kTileKeys * Lds::kChunks,
@@ -1158,8 +1241,8 @@ __device__ __forceinline__ void tile_body(TileLds<T, D, RW>& lds, int it, int pa
     }
     const int ctx = seq_lens[i];
     const int np = kW ? 1 : nparts[i];
-    if constexpr (!kBf16) {  // a split chunk: equal parts
-      if (q_len > kSplitMaxQ) P = chunk_part_len(ctx, np);
+    if constexpr (!kBf16) {
+      if (q_len > kSplitMaxQ) P = chunk_part_len(ctx, np);  // a split chunk
     }
     const int nrows = q_len * rep;
     const bool stream_kv = nrows <= kRows;  // no other pass or row block reads this K / V
@@ -1180,7 +1263,12 @@ __device__ __forceinline__ void tile_body(TileLds<T, D, RW>& lds, int it, int pa
         if (part >= ne) return;
       }
     }
-    const int row0 = rbase + wave * RW;
+    // fp32 items of at most 16 rows (decodes, short verifies): every wavefront
+    // takes the same rows and its own 16 keys of each tile, instead of three
+    // of them waiting for the first; they merge through LDS at the end (100
+    // decodes of up to 2000 keys at head_dim 80: 166 -> 128 us)
+    const bool narrow = !kBf16 && nrows <= RW;
+    const int row0 = narrow ? 0 : rbase + wave * RW;
     const int wave_last = min(nrows - 1, row0 + RW - 1);
     const int kend_wave = row0 < nrows ? min(kend, ctx - q_len + wave_last / rep + 1) : kbeg;
     const int my_row = row0 + col;
@@ -1196,7 +1284,7 @@ __device__ __forceinline__ void tile_body(TileLds<T, D, RW>& lds, int it, int pa
     // Q^T operand of the QK^T product, kept in registers for the whole item
     typename std::conditional<kBf16, bf16x8_t, float>::type qop[kKS];
     {
-      const T* qrow = query + (int64_t)tok * q_stride + (int64_t)head * D;
+      const TIO* qrow = query + (int64_t)tok * q_stride + (int64_t)head * D;
 #pragma unroll
       for (int s = 0; s < kKS; ++s) {
         if constexpr (kBf16) {
@@ -1207,8 +1295,8 @@ __device__ __forceinline__ void tile_body(TileLds<T, D, RW>& lds, int it, int pa
           // step 4 g + e of the product covers k = 16 g + 4 grp + e: a lane's
           // operands of 4 steps are adjacent, in the query as in a K row
           if (s % 4 == 0) {
-            const f32x4_t w = row_ok ? *reinterpret_cast<const f32x4_t*>(qrow + 4 * s + 4 * grp)
-                                     : (f32x4_t){0.f, 0.f, 0.f, 0.f};
+            const f32x4_t w =
+                row_ok ? load4<kLoose>(qrow + 4 * s + 4 * grp) : (f32x4_t){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int e = 0; e < 4; ++e) qop[s + e] = w[e];
           }
@@ -1278,10 +1366,10 @@ __device__ __forceinline__ void tile_body(TileLds<T, D, RW>& lds, int it, int pa
         for (int r = 0; r < kU; ++r) {
           const int kr = min(k0 + kUnitKeys * (kHalves * r + hg), klast);
           const int64_t boff = (int64_t)((uint64_t)blk[r] * blk_elems) + kv_off;
-          pk[r] = load_kv<kNt, Raw>(kc + boff + ((uint32_t)(kr & bs_mask) * (uint32_t)slot_stride +
+          pk[r] = load_kv<kNt, Raw, kLoose>(kc + boff + ((uint32_t)(kr & bs_mask) * (uint32_t)slot_stride +
                                                  k_thr_off));
           const int vkey = min(kr + tk, kend_wg - 1);
-          pv[r] = load_kv<kNt, Raw>(vc + boff +
+          pv[r] = load_kv<kNt, Raw, kLoose>(vc + boff +
                                     ((uint32_t)(vkey & bs_mask) * (uint32_t)slot_stride + tc));
         }
       } else {
@@ -1290,8 +1378,8 @@ __device__ __forceinline__ void tile_body(TileLds<T, D, RW>& lds, int it, int pa
           const int tk = kIdle ? min(tl / Lds::kChunks, kUnitKeys - 1) : tl / Lds::kChunks;
           const int kk = kUnitKeys * (kHalves * r + hg) + tk;
           const int64_t off = row_of(min(k0 + kk, kend_wg - 1)) + (tl % Lds::kChunks) * kCE;
-          pk[r] = load_kv<kNt, Raw>(kc + off);
-          pv[r] = load_kv<kNt, Raw>(vc + off);
+          pk[r] = load_kv<kNt, Raw, kLoose>(kc + off);
+          pv[r] = load_kv<kNt, Raw, kLoose>(vc + off);
         }
       }
     };
@@ -1335,6 +1423,25 @@ __device__ __forceinline__ void tile_body(TileLds<T, D, RW>& lds, int it, int pa
     };
 
     const int ntile = kend_wg > kbeg ? (kend_wg - kbeg + kTileKeys - 1) / kTileKeys : 0;
+    // fp32 PV operands of one key: the d tiles in quads (row m of tile 4 q + e
+    // is dim 64 q + 4 m + e: one 16-byte read of a V row feeds 4 tiles), then a
+    // pair, then a single one
+    auto vread_f = [&](const Lds& b, int key, float (&vd)[kDT]) {
+      if constexpr (!kBf16) {
+        const float* vrow = &b.v[key * Lds::vRow];
+#pragma unroll
+        for (int q = 0; q < kQuads; ++q) {
+          const f32x4_t w = *reinterpret_cast<const f32x4_t*>(vrow + 64 * q + 4 * col);
+#pragma unroll
+          for (int x = 0; x < 4; ++x) vd[4 * q + x] = w[x];
+        }
+        if constexpr (kPair > 0) {
+          const f32x2_t w = *reinterpret_cast<const f32x2_t*>(vrow + 64 * kQuads + 2 * col);
+          vd[4 * kQuads] = w[0], vd[4 * kQuads + 1] = w[1];
+        }
+        if constexpr (kOdd > 0) vd[kDT - 1] = vrow[16 * (kDT - 1) + col];
+      }
+    };
     // one tile of keys k0.. from LDS b into the running softmax and output
     auto compute = [&](const Lds& b, int k0) {
       // ---- S^T = K Q^T for the key subtiles
@@ -1536,42 +1643,73 @@ __device__ __forceinline__ void tile_body(TileLds<T, D, RW>& lds, int it, int pa
           }
         }
       } else {
-        // the d tiles in quads (row m of tile 4 q + e is dim 64 q + 4 m + e: one
-        // 16-byte read of a V row feeds 4 tiles), then a pair, then a single one
-        // (each key's operands are read kLookF keys before their products: left
+        // each key's operands are read kLookF keys before their products (left
         // to itself the compiler reads and waits key by key)
         constexpr int kLookF = 3;
         float vd[kLookF][kDT];
-        auto vread_f = [&](int st, float (&vd)[kDT]) {  // key 16 (st / 4) + 4 grp + st % 4
-          const float* vrow = &b.v[(16 * (st >> 2) + 4 * grp + (st & 3)) * Lds::vRow];
-#pragma unroll
-          for (int q = 0; q < kQuads; ++q) {
-            const f32x4_t w = *reinterpret_cast<const f32x4_t*>(vrow + 64 * q + 4 * col);
-#pragma unroll
-            for (int x = 0; x < 4; ++x) vd[4 * q + x] = w[x];
-          }
-          if constexpr (kPair > 0) {
-            const f32x2_t w = *reinterpret_cast<const f32x2_t*>(vrow + 64 * kQuads + 2 * col);
-            vd[4 * kQuads] = w[0], vd[4 * kQuads + 1] = w[1];
-          }
-          if constexpr (kOdd > 0) vd[kDT - 1] = vrow[16 * (kDT - 1) + col];
-        };
+        auto key_f = [&](int st) { return 16 * (st >> 2) + 4 * grp + (st & 3); };
         constexpr int kReads = kQuads + kPair + kOdd;  // LDS reads of a step
 #pragma unroll
-        for (int st = 0; st < kLookF; ++st) vread_f(st, vd[st]);
+        for (int st = 0; st < kLookF; ++st) vread_f(b, key_f(st), vd[st]);
 #pragma unroll
         for (int st = 0; st < 4 * kST; ++st) {
 #pragma unroll
           for (int u = 0; u < kDT; ++u)
             acc[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(vd[st % kLookF][u], pr[st >> 2][st & 3],
                                                           acc[u], 0, 0, 0);
-          if (st + kLookF < 4 * kST) vread_f(st + kLookF, vd[st % kLookF]);
+          if (st + kLookF < 4 * kST) vread_f(b, key_f(st + kLookF), vd[st % kLookF]);
         }
         __builtin_amdgcn_sched_group_barrier(0x100, kLookF * kReads, 1);
 #pragma unroll
         for (int st = 0; st < 4 * kST; ++st) {
           __builtin_amdgcn_sched_group_barrier(0x008, kDT, 1);
           if (st + kLookF < 4 * kST) __builtin_amdgcn_sched_group_barrier(0x100, kReads, 1);
+        }
+      }
+    };
+    // the same for a narrow item: the wavefront's 16 keys of the tile only
+    auto compute_narrow = [&](const Lds& b, int k0) {
+      if constexpr (!kBf16) {
+        const int kb = 16 * wave;
+        if (k0 + kb >= kend_wave) return;  // wave-uniform
+        AccT s0 = {0.f, 0.f, 0.f, 0.f}, s1 = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int g = 0; g < D / 16; ++g) {
+          const f32x4_t a =
+              *reinterpret_cast<const f32x4_t*>(&b.k[(kb + col) * Lds::kRow + 16 * g + 4 * grp]);
+          s0 = __builtin_amdgcn_mfma_f32_16x16x4f32(a[0], qop[4 * g], s0, 0, 0, 0);
+          s1 = __builtin_amdgcn_mfma_f32_16x16x4f32(a[1], qop[4 * g + 1], s1, 0, 0, 0);
+          s0 = __builtin_amdgcn_mfma_f32_16x16x4f32(a[2], qop[4 * g + 2], s0, 0, 0, 0);
+          s1 = __builtin_amdgcn_mfma_f32_16x16x4f32(a[3], qop[4 * g + 3], s1, 0, 0, 0);
+        }
+        float sc[4], cmax = -__builtin_inff();
+        const int lim = min(qpos + 1, kend) - (k0 + kb + 4 * grp);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          sc[r] = r < lim ? s0[r] + s1[r] : -__builtin_inff();
+          cmax = fmaxf(cmax, sc[r]);
+        }
+        cmax = fmaxf(cmax, __shfl_xor(cmax, 16, 64));
+        cmax = fmaxf(cmax, __shfl_xor(cmax, 32, 64));
+        const float m_new = fmaxf(m_run, cmax * scale_log2);
+        const float alpha = m_new == -__builtin_inff() ? 1.f : exp2_fast(m_run - m_new);
+        const float ref = m_new == -__builtin_inff() ? 0.f : m_new;
+        m_run = m_new;
+        l_part *= alpha;
+#pragma unroll
+        for (int u = 0; u < kDT; ++u) acc[u] *= alpha;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          sc[r] = exp2_fast(fmaf(sc[r], scale_log2, -ref));
+          l_part += sc[r];
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          float vd[kDT];
+          vread_f(b, kb + 4 * grp + e, vd);
+#pragma unroll
+          for (int u = 0; u < kDT; ++u)
+            acc[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(vd[u], sc[e], acc[u], 0, 0, 0);
         }
       }
     };
@@ -1612,7 +1750,9 @@ __device__ __forceinline__ void tile_body(TileLds<T, D, RW>& lds, int it, int pa
       stage(lds, k0, pk, pv);
       __syncthreads();
       if (ti + ahead < ntile) prefetch(k0 + ahead * kTileKeys, pk, pv);  // in flight meanwhile
-      if (k0 < kend_wave) compute(lds, k0);  // else every row of the wave is past its end
+      if (!kBf16 && narrow)
+        compute_narrow(lds, k0);
+      else if (k0 < kend_wave) compute(lds, k0);  // else every row of the wave is past its end
     };
     if constexpr (kDeep) {
       // three tiles in flight (three register sets, the loop unrolled by
@@ -1632,20 +1772,59 @@ __device__ __forceinline__ void tile_body(TileLds<T, D, RW>& lds, int it, int pa
       if (ntile > 0) prefetch(kbeg, pk, pv);
       for (int ti = 0; ti < ntile; ++ti) tile_step(ti, 1, pk, pv);
     }
+    if (!kBf16 && narrow) {
+      // wavefront 0 takes the others' results, lane by lane, and writes
+      if constexpr (!kBf16) {
+        constexpr int kVals = 4 * kDT + 2;
+        static_assert(3 * kVals <= kTileKeys * Lds::kRow / 64, "three wavefronts' values fit the K rows");
+        __syncthreads();  // the last tile is done with the LDS
+        float* buf = lds.k + (wave - 1) * kVals * 64 + lane;
+        if (wave > 0) {
+          buf[0] = m_run, buf[64] = l_part;
+#pragma unroll
+          for (int u = 0; u < kDT; ++u)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) buf[64 * (2 + 4 * u + r)] = acc[u][r];
+        }
+        __syncthreads();
+        if (wave == 0) {
+          const float* src = lds.k + lane;
+          float mw[3], M = m_run;
+#pragma unroll
+          for (int w = 0; w < 3; ++w) mw[w] = src[w * kVals * 64], M = fmaxf(M, mw[w]);
+          auto weight = [&](float m) { return m == -__builtin_inff() ? 0.f : exp2_fast(m - M); };
+          const float w0 = weight(m_run);
+          l_part *= w0, m_run = M;
+#pragma unroll
+          for (int u = 0; u < kDT; ++u) acc[u] *= w0;
+#pragma unroll
+          for (int w = 0; w < 3; ++w) {
+            const float* from = src + w * kVals * 64;
+            const float ww = weight(mw[w]);
+            l_part = fmaf(from[64], ww, l_part);
+#pragma unroll
+            for (int u = 0; u < kDT; ++u)
+#pragma unroll
+              for (int r = 0; r < 4; ++r)
+                acc[u][r] = fmaf(from[64 * (2 + 4 * u + r)], ww, acc[u][r]);
+          }
+        }
+      }
+    }
     // ---- row sums over the lane groups, then write
     float l_row = l_part;
     if constexpr (!kW) l_row += __shfl_xor(l_row, 16, 64);
     l_row += __shfl_xor(l_row, 32, 64);
-    if (row_ok) {
+    if (row_ok && !(narrow && wave > 0)) {
       if (ne == 1) {
         const float inv = l_row > 0.f ? 1.f / l_row : 0.f;
-        T* orow = out + ((int64_t)tok * H + head) * D;
+        TIO* orow = out + ((int64_t)tok * H + head) * D;
         each4([&](int d, float x0, float x1, float x2, float x3) {
           x0 *= inv, x1 *= inv, x2 *= inv, x3 *= inv;
           if constexpr (kBf16)
             *reinterpret_cast<uint2*>(orow + d) = make_uint2(cvt_pk_bf16(x0, x1), cvt_pk_bf16(x2, x3));
           else
-            *reinterpret_cast<float4*>(orow + d) = make_float4(x0, x1, x2, x3);
+            store4<kLoose>(orow + d, (f32x4_t){x0, x1, x2, x3});
         });
       } else {
         // the partial at device scope (written through to the point of
@@ -1681,7 +1860,7 @@ __device__ __forceinline__ void tile_body(TileLds<T, D, RW>& lds, int it, int pa
       __syncthreads();
       if (lds.last) {
         asm volatile("" ::: "memory");  // no load below moves above the arrival
-        merge_tile_rows<T, D, kWv>(
+        merge_tile_rows<TIO, D, kWv, kLoose>(
             out, H, rep, kvh, rbase, min(nrows, rbase + kItemRows), qsl[i], np, ne,
             (int64_t)split_base[i], ml, po, wave, lane);
       }
@@ -1727,10 +1906,13 @@ __device__ __forceinline__ int claimed_item(int64_t c, int stride, int base, int
 // items longest first, so the launch ends on short ones. The counters are
 // zeroed by the plan and, at the end of every run, by the claims that return
 // each queue's last value (below).
-template <typename T, int D, int RW, int kWv, typename TKV = T>
+// T: the products' operands, TKV: cache elements, TIO: query and output
+// elements (T = float over bf16 ones for bf16 head dims other than 64 and 128:
+// everything widened exactly, the weights kept in fp32)
+template <typename T, int D, int RW, int kWv, typename TKV = T, typename TIO = T>
 __global__ void __launch_bounds__(64 * kWv)
 __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 && D <= 64 ? 3 : 2))) attend_tile_kernel(
-    VL_ATTN_PARAMS_KV(T, TKV), const int32_t* __restrict__ hdr, const int32_t* __restrict__ item_off,
+    VL_ATTN_PARAMS_KV(TIO, TKV), const int32_t* __restrict__ hdr, const int32_t* __restrict__ item_off,
     const int32_t* __restrict__ item_seq, int32_t* counters) {
   __shared__ TileLds<T, D, RW> lds;
   __shared__ int claim_lds;
@@ -1755,7 +1937,7 @@ __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 && D <= 64 ? 3 : 2))) attend_t
         __hip_atomic_store(counters + xcd, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       nxt = claimed_item(per_queue + (int64_t)c, kXcds, xcd, n_items);
     }
-    tile_body<T, D, RW, false, kWv, TKV>(lds, it, 0, P, item_off, item_seq, VL_ATTN_ARGS);
+    tile_body<T, D, RW, false, kWv, TKV, TIO>(lds, it, 0, P, item_off, item_seq, VL_ATTN_ARGS);
     __syncthreads();  // the item is done with the LDS; claim_lds has been read
     if (threadIdx.x == 0) claim_lds = nxt;
     __syncthreads();
@@ -2792,11 +2974,11 @@ int do_plan(const Args& a, void* ws, size_t ws_bytes, hipStream_t st) {
   const bool tile = tile_shape(a.dtype, a.D, a.bs);
   // a few bandwidth-kernel items per resident workgroup
   const int target_items = fast ? kItemsPerWg * decode_grid() : 0;
-  const int tile_target = kTileItemsPerWg * tile_grid();
   const int chunk_target = kChunkItemsPerCu * vl_num_cus();
-  const bool wide = tile && a.dtype == VL_DTYPE_BF16;
+  const bool wide = tile && bf16_tile_shape(a.dtype, a.D);
+  const int tile_target = wide ? kTileItemsPerWg * tile_grid() : kTileItemsPerWgF32 * tile_grid();
   auto* plan = a.S <= kPlanThreads * kPlanRegSeqs ? plan_kernel<true> : plan_kernel<false>;
-  plan<<<1, kPlanThreads, 0, st>>>(a.seq_lens, a.qsl, a.S, a.H, a.Hkv, fast, tile, wide,
+  plan<<<1, kPlanThreads, 0, st>>>(a.seq_lens, a.qsl, a.S, a.H / a.Hkv, a.Hkv, fast, tile, wide,
                                    L.cap_rows, target_items, tile_target, chunk_target,
                                    L.hdr, L.gen_off,
                                    L.tile_off, L.nparts, L.split_base, L.wide_off, L.cmb_seq,
@@ -2815,14 +2997,14 @@ int do_plan(const Args& a, void* ws, size_t ws_bytes, hipStream_t st) {
 
 // Workgroups of a tile kernel that are resident at once on the current device
 // (its grid is persistent), cached per device and instantiation.
-template <typename T, int D, int RW, int kWv, typename TKV = T>
+template <typename T, int D, int RW, int kWv, typename TKV = T, typename TIO = T>
 int tile_launch_grid() {
   static int cached[64] = {0};
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) dev = 0;
   if (!cached[dev]) {
     int per_cu = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, attend_tile_kernel<T, D, RW, kWv, TKV>,
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, attend_tile_kernel<T, D, RW, kWv, TKV, TIO>,
                                                      64 * kWv, 0) != hipSuccess ||
         per_cu <= 0)
       per_cu = 2;
@@ -2836,22 +3018,23 @@ int tile_launch_grid() {
 // 32-row items (kWideRows rows) by 8-wavefront workgroups: every staged K/V
 // tile serves 256 rows (prefill chunks 278-300 -> 256-274 us against 4
 // wavefronts); 16-row items by 4.
-template <typename T, int D, int RW, typename TKV = T>
+template <typename T, int D, int RW, typename TKV = T, typename TIO = T>
 int launch_tile_d(const Args& a, const Layout& L, float sl2, hipStream_t st) {
   constexpr int kWv = RW == 32 ? 8 : 4;
-  attend_tile_kernel<T, D, RW, kWv, TKV><<<tile_launch_grid<T, D, RW, kWv, TKV>(), 64 * kWv, 0,
-                                           st>>>(
-      VL_ATTN_LAUNCH_ARGS_KV(T, TKV), L.hdr, RW == 32 ? L.wide_off : L.tile_off,
-      RW == 32 ? L.wide_seq : L.tail_seq, L.hdr + (RW == 32 ? 34 : 26));
+  attend_tile_kernel<T, D, RW, kWv, TKV, TIO>
+      <<<tile_launch_grid<T, D, RW, kWv, TKV, TIO>(), 64 * kWv, 0, st>>>(
+          VL_ATTN_LAUNCH_ARGS_KV(TIO, TKV), L.hdr, RW == 32 ? L.wide_off : L.tile_off,
+          RW == 32 ? L.wide_seq : L.tail_seq, L.hdr + (RW == 32 ? 34 : 26));
   VL_CHECK_LAUNCH();
   return VL_OK;
 }
 
-// The 16-row tile kernel always (short-query and fp32 items); for bf16 also
-// the 32-row kernel when a sequence may have more than kSplitMaxQ queries.
+// The 16-row tile kernel always (short-query and fp32 items); for bf16 head
+// dims 64 and 128 also the 32-row kernel when a sequence may have more than
+// kSplitMaxQ queries.
 template <typename T, typename TKV = T>
 int launch_tile(const Args& a, const Layout& L, float sl2, int max_q, hipStream_t st) {
-  const bool wide = sizeof(T) == 2 && (max_q <= 0 || max_q > kSplitMaxQ);
+  const bool wide = max_q <= 0 || max_q > kSplitMaxQ;
   int rc = VL_OK;
   if constexpr (sizeof(T) == 2) {
     switch (a.D) {
@@ -2863,6 +3046,12 @@ int launch_tile(const Args& a, const Layout& L, float sl2, int max_q, hipStream_
         rc = launch_tile_d<T, 128, 16>(a, L, sl2, st);
         if (!rc && wide) rc = launch_tile_d<T, 128, 32>(a, L, sl2, st);
         return rc;
+      case 16: return launch_tile_d<float, 16, 16, T, T>(a, L, sl2, st);
+      case 32: return launch_tile_d<float, 32, 16, T, T>(a, L, sl2, st);
+      case 48: return launch_tile_d<float, 48, 16, T, T>(a, L, sl2, st);
+      case 80: return launch_tile_d<float, 80, 16, T, T>(a, L, sl2, st);
+      case 96: return launch_tile_d<float, 96, 16, T, T>(a, L, sl2, st);
+      case 112: return launch_tile_d<float, 112, 16, T, T>(a, L, sl2, st);
     }
   } else {
     switch (a.D) {
@@ -2870,6 +3059,9 @@ int launch_tile(const Args& a, const Layout& L, float sl2, int max_q, hipStream_
       case 32: return launch_tile_d<T, 32, 16, TKV>(a, L, sl2, st);
       case 48: return launch_tile_d<T, 48, 16, TKV>(a, L, sl2, st);
       case 64: return launch_tile_d<T, 64, 16, TKV>(a, L, sl2, st);
+      case 80: return launch_tile_d<T, 80, 16, TKV>(a, L, sl2, st);
+      case 96: return launch_tile_d<T, 96, 16, TKV>(a, L, sl2, st);
+      case 112: return launch_tile_d<T, 112, 16, TKV>(a, L, sl2, st);
       case 128: return launch_tile_d<T, 128, 16, TKV>(a, L, sl2, st);
     }
   }
@@ -3082,8 +3274,8 @@ extern "C" int vl_paged_attention_run(void* out, const void* query, int64_t quer
     if (int rc = vl_kv_geom(kv_layout, block_size, num_kv_heads, head_dim, &geom)) return rc;
   int rc = check_args(a, workspace, workspace_bytes, true);
   if (rc || a.S == 0 || a.T == 0) return rc;
-  if (fast_shape(dtype, num_heads, num_kv_heads, head_dim, block_size) ||
-      tile_shape(dtype, head_dim, block_size))
+  if (tile_shape(dtype, head_dim, block_size) &&
+      aligned_tile_dim(dtype == VL_DTYPE_BF16, head_dim))  // (the fast shape is one of these)
     VL_CHECK_ARG((query_stride % 8) == 0 && ((uintptr_t)query & 15) == 0 &&
                      ((uintptr_t)out & 15) == 0 && ((uintptr_t)key_cache & 15) == 0 &&
                      ((uintptr_t)value_cache & 15) == 0,
