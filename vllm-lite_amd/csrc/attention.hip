@@ -2438,20 +2438,6 @@ struct ShortLds {
   float o[REP * D];         // with wo: the workgroup's merged output rows
 };
 
-
-
-
-// A head row of D elements of T as floats (16-byte loads).
-template <typename T, int D>
-__device__ __forceinline__ void load_row(const T* p, float (&r)[D]) {
-  constexpr int VE = 16 / (int)sizeof(T);
-#pragma unroll
-  for (int c = 0; c < D / VE; ++c) {
-    const uint4 v = reinterpret_cast<const uint4*>(p)[c];
-    widen16<T>(v, r + VE * c);
-  }
-}
-
 // T: query and output elements, TKV: cache elements; NW wavefronts.
 // With wo (fp32 T only): instead of its REP output rows the workgroup writes
 // parts[i, g, :] = (its REP x D outputs, as one row) @ wo[g REP D .. (g + 1)
@@ -2530,17 +2516,23 @@ __global__ void __launch_bounds__(64 * NW) attend_short_decode_kernel(
     // 16-byte chunk pc of keys pg + G j, so each load instruction reads G
     // whole rows (a lane per key reads one chunk of 64 rows, 64 cache lines,
     // per instruction: the address work of those loads set the kernel's time)
-    uint4 kraw[Lds::kStageK ? KPL : 1], vraw[KPL];
+    uint4 kraw[KPL], vraw[KPL];
 #pragma unroll
     for (int j = 0; j < KPL; ++j) {
       const int kk = min(pg + G * j, 63);  // past the chunk (or lanes past G NC): weight 0
       const int64_t ro = row_of(min(base + kk, c - 1)) + pc * VE;
-      if constexpr (Lds::kStageK) kraw[j] = *reinterpret_cast<const uint4*>(kg + ro);
+      kraw[j] = *reinterpret_cast<const uint4*>(kg + ro);
       vraw[j] = *reinterpret_cast<const uint4*>(vg + ro);
     }
-    // the lane's key row: through the wavefront's LDS rows, or (fp32 head_dim
-    // 64, whose rows do not fit) straight from the cache
-    float kr[D];
+    // the lane's key: its whole row through the wavefront's LDS rows, or (fp32
+    // head_dim 64, whose rows do not fit: a row is 16 chunks, a key group 16
+    // lanes) every lane multiplies its chunk of the group's 16 keys and a
+    // transposing sum over the 16 lanes leaves key pg + G pc's score with lane
+    // (pg, pc). (A lane per key row straight from the cache read each 64-byte
+    // sector four times, 16 bytes at a time, past what the L1 holds: 32
+    // sequences x 8 heads of up to 1200 keys 32.5 us; this way 17, 5.0 TB/s.)
+    float kr[Lds::kStageK ? D : 1];
+    int my_key = lane;
     if constexpr (Lds::kStageK) {
 #pragma unroll
       for (int j = 0; j < KPL; ++j) {
@@ -2553,14 +2545,29 @@ __global__ void __launch_bounds__(64 * NW) attend_short_decode_kernel(
 #pragma unroll
       for (int cc = 0; cc < NC; ++cc) widen16<TKV>(s.k[wave][lane][cc], kr + VE * cc);
     } else {
-      load_row<TKV, D>(kg + row_of(min(base + lane, c - 1)), kr);
+      static_assert(Lds::kStageK || (NC == 16 && KPL == 16 && sizeof(TKV) == 4),
+                    "a key group is one 16-lane row");
+      my_key = pg + G * pc;
     }
-    const bool valid = base + lane < c;
+    const bool valid = base + my_key < c;
 #pragma unroll
     for (int h = 0; h < REP; ++h) {
       float a = 0.f;
+      if constexpr (Lds::kStageK) {
 #pragma unroll
-      for (int d = 0; d < D; ++d) a = __builtin_fmaf(s.q[h][d], kr[d], a);
+        for (int d = 0; d < D; ++d) a = __builtin_fmaf(s.q[h][d], kr[d], a);
+      } else {
+        const float4 q4 = *reinterpret_cast<const float4*>(&s.q[h][VE * pc]);
+        float part[KPL];
+#pragma unroll
+        for (int j = 0; j < KPL; ++j) {
+          float x[VE];
+          widen16<TKV>(kraw[j], x);
+          part[j] = __builtin_fmaf(
+              x[3], q4.w, __builtin_fmaf(x[2], q4.z, __builtin_fmaf(x[1], q4.y, x[0] * q4.x)));
+        }
+        a = row_transpose_sum16(part, pc);
+      }
       const float sc = valid ? a : -__builtin_inff();
       const float mn = fmaxf(m[h], wave_max_dpp(sc));  // finite: key base is valid
       const float alpha = exp2_fast(m[h] - mn);
@@ -2569,7 +2576,7 @@ __global__ void __launch_bounds__(64 * NW) attend_short_decode_kernel(
 #pragma unroll
       for (int e = 0; e < VE; ++e) acc[h][e] *= alpha;
       m[h] = mn;
-      s.p[wave][h][lane] = p;
+      s.p[wave][h][my_key] = p;
     }
     // the weights the wavefront's other lanes wrote above
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
