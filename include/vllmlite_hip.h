@@ -291,6 +291,15 @@ int vl_linear_rows_parts(float* out, int64_t out_stride, const float* x, int64_t
                          void* stream);
 
 /*
+ * vl_linear_rows over tiled weights for deeper products (k a multiple of 16,
+ * k <= 2048; no row index, no norm; mode VL_LINEAR_STORE or
+ * VL_LINEAR_ACCUMULATE): the down projection of vllmlite/model.py:117 of
+ * models with d_ff above 1024.
+ */
+int vl_linear_rows_deep(float* out, int64_t out_stride, const float* x, int64_t x_stride,
+                        const float* weight, int rows, int k, int n, int mode, void* stream);
+
+/*
  * K6b the QKV projection of a step's rows fused with RoPE and the K/V
  * scatter (vllmlite/model.py:96-103, 109; vllmlite/attention.py:21-37,
  * 47-49): qkv = f(x) @ weight (weight [k, (num_heads + 2 num_kv_heads) *

@@ -1,0 +1,126 @@
+"""The projections of many rows (linear_tile_kernel, chosen from a grid of one
+32-row workgroup per compute unit) and the deep down projection, against
+float64 NumPy, and a model that needs both against the oracle runner."""
+
+import numpy as np
+import pytest
+
+torch = pytest.importorskip("torch")
+
+from helpers import small_cfg  # noqa: E402
+from test_gpu_linear import _close, _ops, _rms, _silu  # noqa: E402
+from test_gpu_runner import PROMPTS, _logit_trace  # noqa: E402
+
+pytestmark = pytest.mark.gpu
+
+
+def _dev(a):
+    return torch.from_numpy(np.ascontiguousarray(a)).cuda()
+
+
+# 32- and 64-row workgroups, a last row block and a last column block that are
+# not full, K below a chunk of 64, a multiple of it and not
+@pytest.mark.parametrize("rows,k,n,mode", [(1400, 1024, 384, "accumulate"), (1000, 496, 1100, "store"),
+                                           (1030, 384, 1152, "store"), (700, 64, 1030, "swiglu"),
+                                           (260, 512, 2048, "swiglu"), (2050, 16, 520, "store")])
+@pytest.mark.parametrize("norm", [False, True])
+def test_many_rows_over_tiled_weights(rows, k, n, mode, norm):
+    o = _ops()
+    rng = np.random.default_rng(rows + k + norm)
+    halves = 2 if mode == "swiglu" else 1
+    x = rng.standard_normal((rows, k)).astype(np.float32)
+    w = (0.05 * rng.standard_normal((k, halves * n))).astype(np.float32)
+    g = (1.0 + 0.1 * rng.standard_normal(k)).astype(np.float32)
+    res = rng.standard_normal((rows, n)).astype(np.float32)
+    y = (_rms(x.astype(np.float64), g.astype(np.float64)) if norm else x.astype(np.float64)) @ w
+    want = {"store": y[:, :n], "accumulate": res + y[:, :n],
+            "swiglu": _silu(y[:, :n]) * y[:, n:] if halves == 2 else None}[mode]
+    out = _dev(res)
+    o.linear_rows(out, _dev(x), o.tile16(_dev(w), halves), _dev(g) if norm else None,
+                  mode={"store": o.LINEAR_STORE, "accumulate": o.LINEAR_ACCUMULATE,
+                        "swiglu": o.LINEAR_SWIGLU}[mode])
+    torch.cuda.synchronize()
+    _close(out.cpu().numpy(), want)
+
+
+@pytest.mark.parametrize("rows", [1, 16, 33, 1100])
+@pytest.mark.parametrize("k,n", [(16, 512), (1040, 40), (2048, 512)])
+def test_deep_projection(rows, k, n):
+    o = _ops()
+    rng = np.random.default_rng(rows + k)
+    x = rng.standard_normal((rows, k)).astype(np.float32)
+    w = (0.02 * rng.standard_normal((k, n))).astype(np.float32)
+    res = rng.standard_normal((rows, n)).astype(np.float32)
+    wt = o.tile16(_dev(w))
+    out, acc = torch.full((rows, n), float("nan"), device="cuda"), _dev(res)
+    o.linear_rows_deep(out, _dev(x), wt)
+    o.linear_rows_deep(acc, _dev(x), wt, mode=o.LINEAR_ACCUMULATE)
+    torch.cuda.synchronize()
+    want = x.astype(np.float64) @ w.astype(np.float64)
+    _close(out.cpu().numpy(), want)
+    _close(acc.cpu().numpy(), res + want)
+    with pytest.raises(RuntimeError):  # deeper than the kernel
+        o.linear_rows_deep(out, torch.zeros(rows, 2064, device="cuda"),
+                           torch.zeros(-(-n // 16), 2064, 16, device="cuda"))
+
+
+@pytest.mark.parametrize("layout", ["token", "head"])
+@pytest.mark.parametrize("cache", [torch.float32, torch.bfloat16])
+def test_many_rows_qkv_equals_projection_then_rope(layout, cache):
+    """Rows gathered by index with placeholders, copied to x_out, the record
+    copied too: the same bits as the projection of the gathered rows followed
+    by vl_rope_and_cache."""
+    o = _ops()
+    H, Hkv, D, k, rows = 8, 4, 48, 384, 1000
+    n = (H + 2 * Hkv) * D
+    rng = np.random.default_rng(3)
+    table = _dev(rng.standard_normal((261, k)).astype(np.float32))
+    prev = _dev(rng.integers(0, 261, 12).astype(np.int32))
+    ids_np = rng.integers(0, 261, rows).astype(np.int32)
+    ids_np[[0, 500, 999]] = [-1, -12, -13]  # -13: past num_prev -> id 0
+    ids = _dev(ids_np)
+    w = o.tile16(_dev((0.05 * rng.standard_normal((k, n))).astype(np.float32)))
+    g = _dev((1.0 + 0.1 * rng.standard_normal(k)).astype(np.float32))
+    pos = _dev(rng.integers(0, 64, rows).astype(np.int32))
+    slots = rng.permutation(1008)[:rows].astype(np.int32)
+    slots[::7] = -1
+    slot = _dev(slots)
+    ang = rng.standard_normal((64, D // 2)).astype(np.float32)
+    cos, sin = _dev(np.cos(ang)), _dev(np.sin(ang))
+    shape = (63, Hkv, 16, D) if layout == "head" else (1008, Hkv, D)
+    kc1, vc1, kc2, vc2 = (torch.zeros(shape, device="cuda", dtype=cache) for _ in range(4))
+    q1, q2 = torch.empty((rows, H, D), device="cuda"), torch.empty((rows, H * D), device="cuda")
+    x_out = torch.full((rows, k), float("nan"), device="cuda")
+    rec = torch.arange(200001, dtype=torch.int32).pin_memory()
+    rec_dst = torch.zeros(200001, dtype=torch.int32, device="cuda")
+    o.qkv_rope_cache(q2, kc2, vc2, table, w, g, pos, slot, cos, sin, H, Hkv, D, row_index=ids,
+                     x_out=x_out, prev_ids=prev, record=(rec, rec_dst))
+    o.resolve_tokens(ids, prev)
+    x = table[ids.long()].contiguous()
+    qkv = torch.empty((rows, n), device="cuda")
+    o.linear_rows(qkv, x, w, g, mode=o.LINEAR_STORE)
+    o.rope_and_cache(qkv, q1, kc1, vc1, pos, slot, cos, sin, H, Hkv, D)
+    torch.cuda.synchronize()
+    assert torch.equal(q1.view(rows, -1), q2) and torch.equal(x_out, x)
+    assert torch.equal(kc1, kc2) and torch.equal(vc1, vc2)
+    assert torch.equal(rec_dst.cpu(), rec)
+
+
+@pytest.mark.parametrize("shape", [dict(n_heads=4, n_kv_heads=4, d_model=128, d_ff=1040),
+                                   dict(n_heads=8, n_kv_heads=8, d_model=512, d_ff=2048),
+                                   dict(n_heads=8, n_kv_heads=4, d_model=512, d_ff=512)])
+def test_deeper_models_match_the_oracle_runner(shape):
+    """Every step's logits of models whose down projection is deeper than
+    vl_linear_rows takes, or whose decode steps keep wo out of the attention
+    launch: within 2e-4 of each row's largest logit, as the other shapes."""
+    from oracle.runner import NumpyRunner
+    from vllmlite_amd.hip_runner import HipRunner
+    cfg = small_cfg(layers=2)
+    for f, v in shape.items():
+        setattr(cfg.model, f, v)
+    got = _logit_trace(HipRunner, cfg, PROMPTS, 6)
+    want = _logit_trace(NumpyRunner, cfg, PROMPTS, 6)
+    assert len(got) == len(want)
+    for (g, dec), (w, _) in zip(got, want):
+        scale = np.abs(w).max(axis=-1, keepdims=True)
+        assert np.all(np.abs(g - w) <= 2e-4 * scale), f"decode step {dec}"

@@ -437,6 +437,260 @@ __global__ void __launch_bounds__(64 * kLinWaves) linear_rows_kernel(
   }
 }
 
+// The same projections for many rows (prefill steps): a workgroup of 4
+// wavefronts computes 16 RS rows x 64 columns, a wavefront 16 of them (one
+// weight tile). x goes through LDS, kTileK of its columns at a time in two
+// buffers, so that the workgroup reads each row once for its 64 columns; the
+// weights of a chunk go straight to registers, a chunk ahead. Each 16-k
+// group is its own MFMA chain, added to the running sums when the chunk ends:
+// chains of 4 products, whatever K is, so that the sums are as close to the
+// 64-bit ones as linear_rows_kernel's (relative error 1.1e-7 at K 384, 1.4e-7
+// at 2048; chains of 8 products 1.3e-7 and 1.5e-7, one chain over all of K
+// 3.5e-7 and 8.1e-7). x * norm_w is staged; the rows' sums of
+// squares are taken as they are staged, and the 1 / rms applied at the end.
+// Bound by the fp32 matrix pipe: per 16-k group a wavefront issues 4 RS
+// products of 32 cycles per weight slice against RS 16-byte LDS reads and one
+// 16-byte load.
+constexpr int kTileK = 64;
+constexpr int kTileWaves = 4;
+
+template <int MODE, bool NORM, int RS>
+__global__ void __launch_bounds__(64 * kTileWaves) linear_tile_kernel(
+    float* __restrict__ out, int64_t ldo, const float* __restrict__ x, int64_t ldx,
+    const float* __restrict__ w, int64_t up_off, const float* __restrict__ norm_w, float eps, int M,
+    int K, int N, const RopeCache rc, const int32_t* __restrict__ row_index,
+    const int32_t* __restrict__ prev_ids, int64_t num_prev, float* __restrict__ x_out) {
+  constexpr int kSlices = MODE == 2 ? 2 : 1;
+  constexpr int kRows = 16 * RS, kLd = kTileK + 4;  // odd number of 16-byte chunks: no conflicts
+  constexpr int kG = kTileK / 16;
+  __shared__ float xs[2][kRows * kLd];
+  __shared__ float rms_s[NORM ? kRows : 1];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int m = lane & 15, j = lane >> 4;
+  const int r0 = blockIdx.y * kRows;
+  const int ntile = (N + kCols - 1) / kCols;
+  const int ct = blockIdx.x * kTileWaves + wave;
+  const bool live = ct < ntile;
+  const int c0 = ct * kCols;
+  // staging: thread t takes 16-byte chunk t % 16 of rows t / 16 + 16 i
+  const int sr = tid >> 4, sk = (tid & 15) * 4;
+  const float* xrow[RS];
+#pragma unroll
+  for (int i = 0; i < RS; ++i) {
+    int64_t row = min(r0 + sr + 16 * i, M - 1);
+    if (row_index) {
+      row = row_index[row];
+      if (row < 0) {  // -(1 + i): the previous step's id of its row i
+        const int64_t q = -row - 1;
+        row = prev_ids && q < num_prev ? prev_ids[q] : 0;
+      }
+    }
+    xrow[i] = x + row * ldx;
+  }
+  const float4* wt = reinterpret_cast<const float4*>(w + (int64_t)(live ? ct : 0) * K * kCols) + lane;
+  const float4* wt2 = reinterpret_cast<const float4*>(w + (kSlices > 1 ? up_off : 0) +
+                                                      (int64_t)(live ? ct : 0) * K * kCols) + lane;
+  const int ng = K / 16, nchunk = (K + kTileK - 1) / kTileK;
+  float4 px[RS], pg, wv[kSlices][kG];
+  // loads of chunk c; columns past K repeat the last 16-k group (their weights
+  // are zeroed below)
+  auto load_x = [&](int c) {
+    const int k = min(c * kTileK + sk, K - 4);
+#pragma unroll
+    for (int i = 0; i < RS; ++i) px[i] = *reinterpret_cast<const float4*>(xrow[i] + k);
+    if constexpr (NORM) pg = *reinterpret_cast<const float4*>(norm_w + k);
+  };
+  auto load_w = [&](int c, float4 (&v)[kSlices][kG]) {
+#pragma unroll
+    for (int g = 0; g < kG; ++g) {
+      const int gg = min(c * kG + g, ng - 1);
+      v[0][g] = wt[gg * 64];
+      if constexpr (kSlices > 1) v[1][g] = wt2[gg * 64];
+    }
+  };
+  float ss[RS];
+#pragma unroll
+  for (int i = 0; i < RS; ++i) ss[i] = 0.f;
+  auto stage = [&](int c, float* buf) {
+    const bool in = c * kTileK + sk < K;
+#pragma unroll
+    for (int i = 0; i < RS; ++i) {
+      float4 v = px[i];
+      if constexpr (NORM) {
+        const float q = ((v.x * v.x + v.y * v.y) + v.z * v.z) + v.w * v.w;
+        ss[i] += in ? q : 0.f;
+        v = make_float4(v.x * pg.x, v.y * pg.y, v.z * pg.z, v.w * pg.w);
+      }
+      if (!in) v = make_float4(0.f, 0.f, 0.f, 0.f);
+      *reinterpret_cast<float4*>(&buf[(sr + 16 * i) * kLd + sk]) = v;
+    }
+  };
+  f32x4_t tot[kSlices][RS];
+#pragma unroll
+  for (int s = 0; s < kSlices; ++s)
+#pragma unroll
+    for (int r = 0; r < RS; ++r) tot[s][r] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+
+  // chunk c from its LDS buffer and the weights cur, the loads of chunk c + 1
+  // (the last chunk repeats its own) in flight meanwhile
+  auto step = [&](int c, float4 (&cur)[kSlices][kG], float4 (&next)[kSlices][kG]) {
+    const int cn = min(c + 1, nchunk - 1);
+    load_x(cn);
+    load_w(cn, next);
+    __builtin_amdgcn_sched_barrier(0);  // they stay ahead of the products
+    const float* buf = xs[c & 1];
+    f32x4_t acc[kG][kSlices][RS];
+#pragma unroll
+    for (int g = 0; g < kG; ++g) {
+#pragma unroll
+      for (int s = 0; s < kSlices; ++s)
+#pragma unroll
+        for (int r = 0; r < RS; ++r) acc[g][s][r] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+      f32x4_t a[RS];
+#pragma unroll
+      for (int r = 0; r < RS; ++r)
+        a[r] = *reinterpret_cast<const f32x4_t*>(&buf[(16 * r + m) * kLd + 16 * g + 4 * j]);
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int s = 0; s < kSlices; ++s) {
+          const float4 q = cur[s][g];
+          const float bw = e == 0 ? q.x : e == 1 ? q.y : e == 2 ? q.z : q.w;
+#pragma unroll
+          for (int r = 0; r < RS; ++r)
+            acc[g][s][r] =
+                __builtin_amdgcn_mfma_f32_16x16x4f32(a[r][e], bw, acc[g][s][r], 0, 0, 0);
+        }
+    }
+#pragma unroll
+    for (int s = 0; s < kSlices; ++s)
+#pragma unroll
+      for (int r = 0; r < RS; ++r) tot[s][r] += (acc[0][s][r] + acc[1][s][r]) + (acc[2][s][r] + acc[3][s][r]);
+    __builtin_amdgcn_sched_barrier(0);
+    // (after the last chunk too, unread: under a condition the compiler would
+    // move the loads of x down to it)
+    stage(c + 1, xs[(c + 1) & 1]);
+    __syncthreads();
+  };
+  if (x_out && blockIdx.x == 0) {  // layer 0 keeps the rows it gathers
+#pragma unroll
+    for (int i = 0; i < RS; ++i) {
+      const int row = r0 + sr + 16 * i;
+      for (int k = sk; k < K && row < M; k += kTileK)
+        *reinterpret_cast<float4*>(x_out + (int64_t)row * K + k) =
+            *reinterpret_cast<const float4*>(xrow[i] + k);
+    }
+  }
+  float4 wn[kSlices][kG];
+  load_x(0);
+  load_w(0, wv);
+  stage(0, xs[0]);
+  __syncthreads();
+  for (int c = 0; c < nchunk; c += 2) {
+    step(c, wv, wn);
+    if (c + 1 < nchunk) step(c + 1, wn, wv);
+  }
+  if constexpr (NORM) {
+    // the 16 lanes of a row hold its sum of squares
+#pragma unroll
+    for (int i = 0; i < RS; ++i) {
+      float q = ss[i];
+      q += VL_DPP(0.f, q, 0xB1, 0xF);   // quad_perm [1, 0, 3, 2]
+      q += VL_DPP(0.f, q, 0x4E, 0xF);   // quad_perm [2, 3, 0, 1]
+      q += VL_DPP(0.f, q, 0x141, 0xF);  // row_half_mirror
+      q += VL_DPP(0.f, q, 0x140, 0xF);  // row_mirror
+      if ((tid & 15) == 0) rms_s[sr + 16 * i] = sqrtf(q / (float)K + eps);
+    }
+    __syncthreads();
+  }
+  // ---- lane (m, j) holds rows 16 r + 4 j + i of column c0 + m
+  const int col = c0 + m;
+  const int qd = rc.nh * rc.hd, kd = rc.nkv * rc.hd;  // MODE 3: the q and k columns
+  const int base = MODE != 3 ? 0 : col < qd ? col : col < qd + kd ? col - qd : col - qd - kd;
+  const int head = MODE == 3 ? base / rc.hd : 0, hcol = MODE == 3 ? base - head * rc.hd : 0;
+#pragma unroll
+  for (int r = 0; r < RS; ++r) {
+    float v[kSlices][4], old[4], ec[4], es[4];
+    int slot[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {  // the rows' reads together
+      const int row = min(r0 + 16 * r + 4 * j + i, M - 1);
+      if constexpr (MODE == 1) old[i] = live && col < N ? out[(int64_t)row * ldo + col] : 0.f;
+      if constexpr (MODE == 3) {
+        slot[i] = rc.slots[row];
+        const int64_t tab = (int64_t)rc.positions[row] * (rc.hd >> 1) + (hcol >> 1);
+        const bool rot = live && col < qd + kd;
+        ec[i] = rot ? rc.cos_t[tab] : 0.f;
+        es[i] = rot ? rc.sin_t[tab] : 0.f;
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int lr = 16 * r + 4 * j + i, row = r0 + lr;
+#pragma unroll
+      for (int s = 0; s < kSlices; ++s) v[s][i] = NORM ? tot[s][r][i] / rms_s[lr] : tot[s][r][i];
+      float partner = 0.f;
+      if constexpr (MODE == 3) partner = VL_DPP(0.f, v[0][i], 0xB1, 0xF);  // column c ^ 1
+      if (!live || col >= N || row >= M) continue;
+      if constexpr (MODE == 0) {
+        out[(int64_t)row * ldo + col] = v[0][i];
+      } else if constexpr (MODE == 1) {
+        out[(int64_t)row * ldo + col] = old[i] + v[0][i];
+      } else if constexpr (MODE == 2) {
+        out[(int64_t)row * ldo + col] = silu_times_f32(v[0][i], v[1][i]);
+      } else if (col < qd + kd) {
+        float oe, oo;
+        const bool odd = hcol & 1;
+        rotate_pair_f32(odd ? partner : v[0][i], odd ? v[0][i] : partner, ec[i], es[i], &oe, &oo);
+        const float val = odd ? oo : oe;
+        if (col < qd)
+          rc.q_out[(int64_t)row * qd + col] = val;
+        else if (slot[i] >= 0)
+          store_cache(rc.kc, rc.geom.at(slot[i], head) + hcol, val, rc.kv_dtype);
+      } else if (slot[i] >= 0) {
+        store_cache(rc.vc, rc.geom.at(slot[i], head) + hcol, v[0][i], rc.kv_dtype);
+      }
+    }
+  }
+  if constexpr (MODE == 3) {  // the step's record
+    const int64_t grid_threads = (int64_t)gridDim.x * gridDim.y * (64 * kTileWaves);
+    for (int64_t g = ((int64_t)blockIdx.y * gridDim.x + blockIdx.x) * (64 * kTileWaves) + tid;
+         g < rc.rec_n; g += grid_threads)
+      rc.rec_dst[g] = rc.rec_src[g];
+  }
+}
+
+template <int MODE, bool NORM>
+int launch_tiles(float* out, int64_t ldo, const float* x, int64_t ldx, const float* w,
+                 const float* norm_w, float eps, int M, int K, int N, hipStream_t st,
+                 const int32_t* row_index, const RopeCache& rc, float* x_out,
+                 const int32_t* prev_ids, int64_t num_prev) {
+  const int ntile = (N + kCols - 1) / kCols, cb = (ntile + kTileWaves - 1) / kTileWaves;
+  const int64_t up_off = MODE == 2 ? (int64_t)ntile * K * kCols : 0;
+  // 64-row workgroups while they fill two rounds of the chip, else 32-row ones
+  const bool tall = (int64_t)cb * ((M + 63) / 64) >= 2 * (int64_t)vl_num_cus();
+  if (tall)
+    linear_tile_kernel<MODE, NORM, 4><<<dim3(cb, (M + 63) / 64), 64 * kTileWaves, 0, st>>>(
+        out, ldo, x, ldx, w, up_off, norm_w, eps, M, K, N, rc, row_index, prev_ids, num_prev, x_out);
+  else
+    linear_tile_kernel<MODE, NORM, 2><<<dim3(cb, (M + 31) / 32), 64 * kTileWaves, 0, st>>>(
+        out, ldo, x, ldx, w, up_off, norm_w, eps, M, K, N, rc, row_index, prev_ids, num_prev, x_out);
+  VL_CHECK_LAUNCH();
+  return VL_OK;
+}
+
+// Whether M rows over a tiled weight of N columns take the kernel above: from a
+// grid of one 32-row workgroup per compute unit on. Below, the 8 wavefronts
+// that linear_rows_kernel puts on each 16 x 16 output split K and finish
+// sooner: K 2048, N 512 at 512 rows (128 workgroups) 22.9 against 29.2 us, at
+// 1024 rows 41.9 against 29.6; K 512, N 2 x 2048 (SwiGLU) at 256 rows (256
+// workgroups) 20.3 against 17.2, at 2048 rows 150 against 88; K 512, N 1536 at
+// 1024 rows 32.5 against 21.4.
+inline bool takes_tiles(int M, int N) {
+  const int64_t cb = ((N + kCols - 1) / kCols + kTileWaves - 1) / kTileWaves;
+  return cb * ((M + 31) / 32) >= vl_num_cus();
+}
+
 // Row tiles per workgroup: 1 while the grid is at most one round of two
 // workgroups per CU (the kernel is latency-bound there, so tiles run side by
 // side); beyond that doubled, up to kSubMax, while the grid keeps at
@@ -470,6 +724,11 @@ int launch(float* out, int64_t ldo, const float* x, int64_t ldx, const float* w,
            const int32_t* row_index, const RopeCache& rc = RopeCache{}, float* x_out = nullptr,
            const int32_t* prev_ids = nullptr, int64_t num_prev = 0,
            const float* x_parts = nullptr, const ArgmaxOut& am = ArgmaxOut{}) {
+  if constexpr (MODE != 4 && NP == 0) {
+    if (tiles && takes_tiles(M, N))
+      return launch_tiles<MODE, NORM>(out, ldo, x, ldx, w, norm_w, eps, M, K, N, st, row_index, rc,
+                                      x_out, prev_ids, num_prev);
+  }
   const int ntile = (N + kCols - 1) / kCols;
   const int rt = row_tile(M, N);
   const int row_tiles = (M + rt - 1) / rt;
@@ -480,7 +739,7 @@ int launch(float* out, int64_t ldo, const float* x, int64_t ldx, const float* w,
     linear_rows_kernel<MODE, NORM, KMAX, true, NP><<<grid, 64 * kLinWaves, 0, st>>>(
         out, ldo, x, ldx, w, 0, up_off, norm_w, eps, M, K, N, rc, row_index, prev_ids, num_prev,
         x_out, nsub, rt, x_parts, am);
-  } else if constexpr (NP == 0 && MODE != 4) {
+  } else if constexpr (NP == 0 && MODE != 4 && KMAX <= 1024) {
     const int64_t up_off = MODE == 2 ? N : 0;
     linear_rows_kernel<MODE, NORM, KMAX, false><<<grid, 64 * kLinWaves, 0, st>>>(
         out, ldo, x, ldx, w, ldw, up_off, norm_w, eps, M, K, N, rc, row_index, prev_ids,
@@ -546,6 +805,27 @@ extern "C" int vl_linear_rows(float* out, int64_t out_stride, const float* x, in
       return nrm ? VL_LINEAR_K(2, true) : VL_LINEAR_K(2, false);
   }
 #undef VL_LINEAR_K
+}
+
+extern "C" int vl_linear_rows_deep(float* out, int64_t out_stride, const float* x,
+                                   int64_t x_stride, const float* weight, int rows, int k, int n,
+                                   int mode, void* stream) {
+  VL_CHECK_ARG(rows >= 0 && rows <= kRowsLimit, "rows must be in 0..%d", kRowsLimit);
+  VL_CHECK_ARG(mode == VL_LINEAR_STORE || mode == VL_LINEAR_ACCUMULATE, "bad mode %d", mode);
+  VL_CHECK_ARG(k > 0 && k % 16 == 0 && k <= 2048, "k must be a multiple of 16, at most 2048");
+  VL_CHECK_ARG(n > 0, "n must be positive");
+  if (rows == 0) return VL_OK;
+  VL_CHECK_ARG(out && x && weight, "null pointer");
+  VL_CHECK_ARG((((uintptr_t)x) & 15) == 0 && x_stride % 4 == 0 && x_stride >= k,
+               "x must be 16-byte aligned with a row stride that is a multiple of 4");
+  VL_CHECK_ARG(out_stride >= n, "row stride too small");
+  VL_CHECK_ARG((((uintptr_t)weight) & 15) == 0, "tiled weight must be 16-byte aligned");
+  hipStream_t st = (hipStream_t)stream;
+  if (mode == VL_LINEAR_STORE)
+    return launch<0, false, 2048>(out, out_stride, x, x_stride, weight, 0, true, nullptr, 0.f, rows,
+                                  k, n, st, nullptr);
+  return launch<1, false, 2048>(out, out_stride, x, x_stride, weight, 0, true, nullptr, 0.f, rows,
+                                k, n, st, nullptr);
 }
 
 extern "C" int vl_qkv_rope_cache(float* q_out, void* key_cache, void* value_cache,

@@ -59,9 +59,19 @@ from .runner import ModelRunner
 
 
 # steps of at most this many token rows run the fused projection kernels
-# (vl_linear_rows, vl_qkv_rope_cache: 16-row tiles, norm / residual / SwiGLU /
-# RoPE + scatter inside); larger ones hipBLASLt GEMMs and separate launches
+# (vl_linear_rows, vl_qkv_rope_cache: norm / residual / SwiGLU / RoPE + scatter
+# inside); larger ones hipBLASLt GEMMs and separate launches (a 2048-token step
+# of the default model: 1747 us, by the fused kernels 1813)
 FUSED_ROWS_MAX = 1024
+# decode steps with wo inside the attention launch (one partial row per KV
+# head, summed again by every workgroup of gate|up): up to this many rows and
+# this d_model. The partial rows and the wo columns an attention workgroup
+# multiplies by grow with both: d_model 384, 8 heads over 4 or 8: 16 rows 190
+# and 198 us per step against 197 and 199 with wo in a launch of its own, 32 rows
+# 229 and 253 against 223 and 231; d_model 512 (6 layers, d_ff 2048, 8 over 8):
+# 4 rows 245 against 216, 16 rows 264 against 235, 32 rows 376 against 346
+FUSED_WO_ROWS = 16
+FUSED_WO_D_MODEL = 384
 
 
 def _bucket(n: int, floor: int) -> int:
@@ -145,6 +155,14 @@ def fused_rows_supported(mc) -> bool:
     every step and keep no tiled weight copies."""
     return (mc.d_model % 16 == 0 and mc.d_ff % 16 == 0 and mc.d_model <= 512
             and mc.d_ff <= 1024)
+
+
+def rows_kernels_supported(mc) -> bool:
+    """Whether every projection of the model has a fused kernel: the shapes of
+    fused_rows_supported, and those whose down projection is deeper than
+    vl_linear_rows takes (vl_linear_rows_deep)."""
+    return (mc.d_model % 16 == 0 and mc.d_ff % 16 == 0 and mc.d_model <= 512
+            and mc.d_ff <= ops.LINEAR_DEEP_K)
 
 
 class _Shape:
@@ -286,7 +304,7 @@ class HipRunner(ModelRunner):
             self.stream = torch.cuda.Stream(self.device)
             w = weights if weights is not None else model_weights(mc)
             self.w = pack_weights(mc, w, torch, self.device)
-            self._fused_rows = fused_rows_supported(mc)
+            self._fused_rows = rows_kernels_supported(mc)
             self.fused_rows_max = FUSED_ROWS_MAX
             if self._fused_rows:
                 tile_weights(self.w, ops.tile16, torch)
@@ -306,7 +324,7 @@ class HipRunner(ModelRunner):
             # decode steps of <= 16 sequences as one launch, where a kernel exists
             self._step = None
             self.one_launch_steps = 0
-            if (one_launch_decode and self._fused_rows and ops.decode_step_supported(
+            if (one_launch_decode and fused_rows_supported(mc) and ops.decode_step_supported(
                     mc.d_model, mc.n_heads, mc.n_kv_heads, mc.d_ff, kv, mc.max_seq_len)):
                 self._step = ops.DecodeStep(self.w, self.device)
                 self._exec_ids_host = torch.zeros(ops.DECODE_STEP_ROWS + 1, dtype=torch.int32,
@@ -332,7 +350,7 @@ class HipRunner(ModelRunner):
             self.H, self.Hkv, self.hd, self.block_size, 1, mc.max_seq_len)
         # decode steps with wo inside the attention launch (vl_decode_attention_wo)
         self._fused_wo = (self._short_decode and self._fused_rows and self.Hkv in (1, 2, 4, 8)
-                          and mc.d_model <= 512 and fused_wo)
+                          and mc.d_model <= FUSED_WO_D_MODEL and fused_wo)
 
     def __del__(self):
         # the submission thread may still hold launches of this runner's graphs
@@ -627,6 +645,11 @@ class HipRunner(ModelRunner):
             ops.paged_attention_run(attn, q, kc, vc, bt, lens, qsl, self.scale, self.block_size,
                                     self._ws)
 
+    def _down(self, x, act, L) -> None:
+        """The down projection, added to the residual x."""
+        down = ops.linear_rows if self.model_cfg.d_ff <= 1024 else ops.linear_rows_deep
+        down(x, act, L["w_down_t"], mode=ops.LINEAR_ACCUMULATE)
+
     def _lm_head(self, s: _Shape, x, lidx, ids_host) -> None:
         """The final RMSNorm and lm_head of the logits rows x[lidx] with their
         argmax (vl_linear_rows_argmax: ids from the same launch)."""
@@ -660,7 +683,7 @@ class HipRunner(ModelRunner):
         launch (one partial row per KV head) and the residual add in gate|up's
         prologue: four launches per layer."""
         W, Tb, Rb = self.w, s.Tb, s.Rb
-        if s.decode and self._fused_wo:
+        if s.decode and self._fused_wo and Tb <= FUSED_WO_ROWS:
             self._forward_decode_wo(s, x, q, act, lidx, qsl, lens, bt, ids_host, rec_host)
             return
         pos = self._meta[s.pos:s.pos + Tb]
@@ -676,7 +699,7 @@ class HipRunner(ModelRunner):
             self._attend(s, attn, q, kc, vc, bt, lens, qsl)
             ops.linear_rows(x, attn.view(Tb, -1), L["wo_t"], mode=ops.LINEAR_ACCUMULATE)
             ops.linear_rows(act, x, L["w_gate_up_t"], L["ffn_norm"], mode=ops.LINEAR_SWIGLU)
-            ops.linear_rows(x, act, L["w_down_t"], mode=ops.LINEAR_ACCUMULATE)
+            self._down(x, act, L)
         self._lm_head(s, x, lidx, ids_host)
 
     def _forward_decode_wo(self, s: _Shape, x, q, act, lidx, qsl, lens, bt, ids_host,
@@ -703,7 +726,7 @@ class HipRunner(ModelRunner):
             ops.decode_attention_wo(parts, q, kc, vc, bt, lens, qsl, self.scale,
                                     self.block_size, L["wo"], mc.max_seq_len)
             ops.linear_rows_parts(act, xa, parts, L["w_gate_up_t"], L["ffn_norm"], x_out=xb)
-            ops.linear_rows(xb, act, L["w_down_t"], mode=ops.LINEAR_ACCUMULATE)
+            self._down(xb, act, L)
             xa, xb = xb, xa
         self._lm_head(s, xa, lidx, ids_host)
 

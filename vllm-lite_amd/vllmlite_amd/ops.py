@@ -69,6 +69,8 @@ SIGNATURES = {
     "vl_argmax_rows": (_i32, [_c_void_p, _i64, _i64, _i32, _c_void_p, _c_void_p, _c_void_p]),
     "vl_linear_rows": (_i32, [_c_void_p, _i64, _c_void_p, _i64, _c_void_p, _c_void_p, _i64,
                               _c_void_p, _f32, _i32, _i32, _i32, _i32, _c_void_p]),
+    "vl_linear_rows_deep": (_i32, [_c_void_p, _i64, _c_void_p, _i64, _c_void_p, _i32, _i32, _i32,
+                                   _i32, _c_void_p]),
     "vl_qkv_rope_cache": (_i32, [_c_void_p, _c_void_p, _c_void_p, _c_void_p, _i64, _c_void_p,
                                  _c_void_p, _i64,
                                  _c_void_p, _c_void_p, _i64, _i32, _c_void_p, _f32, _c_void_p,
@@ -516,6 +518,24 @@ def linear_rows(out: torch.Tensor, x: torch.Tensor, weight: torch.Tensor,
                                 _ptr(weight), wstride, _ptr(norm_weight), float(eps), rows, k, n,
                                 mode | (LINEAR_TILES16 if tiles else 0), _stream()),
            "vl_linear_rows")
+
+
+LINEAR_DEEP_K = 2048  # k of vl_linear_rows_deep
+
+
+def linear_rows_deep(out: torch.Tensor, x: torch.Tensor, weight: torch.Tensor,
+                     mode: int = LINEAR_STORE) -> None:
+    """out (= or +=) x @ weight for fp32 rows, weight in 16-column tiles, k up to
+    LINEAR_DEEP_K (vl_linear_rows_deep)."""
+    rows, k = x.shape
+    n = out.shape[1]
+    for t in (out, x, weight):
+        _need(t.dtype == torch.float32 and t.stride(-1) == 1, "fp32 row-major tensors required")
+    _need(out.shape[0] == rows, "shape mismatch")
+    tiles, _ = _weight_layout(weight, k, n, 1)
+    _need(tiles, "weight must be in 16-column tiles")
+    _check(lib().vl_linear_rows_deep(_ptr(out), out.stride(0), _ptr(x), x.stride(0), _ptr(weight),
+                                     rows, k, n, mode, _stream()), "vl_linear_rows_deep")
 
 
 def qkv_rope_cache(q_out: torch.Tensor, key_cache: torch.Tensor, value_cache: torch.Tensor,
