@@ -103,3 +103,24 @@ def test_widened_head_dims_over_an_fp8_cache(D):
     want = oracle_attention(dict(b, k_cache=fp8_e4m3_decode(enc["k_cache"]),
                                  v_cache=fp8_e4m3_decode(enc["v_cache"])))
     check(to_np(out), want, "f32")
+
+
+@pytest.mark.parametrize("seqs", [[(1, 1)], [(1, 127), (1, 128), (1, 129)], [(1, 8192)],
+                                  [(1, 255 + 64 * i) for i in range(24)]])
+@pytest.mark.parametrize("small_ws", [False, True])
+def test_short_decode_batches_of_the_bandwidth_kernel(seqs, small_ws):
+    """Few items: ranges of 128 tokens, doubled to 256 from half a compute
+    unit's worth of items on; contexts around a range's end."""
+    b = make_batch(seqs, 32, 8, 128, 16, seed=len(seqs))
+    ws = ops().lib().vl_paged_attention_min_workspace(len(seqs)) if small_ws else None
+    check(run_attention(b, "bf16", ws_bytes=ws), expected(b, "bf16"), "bf16")
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("seqs", [[(17, 17), (400, 900)], [(16, 900), (17, 300)], [(5, 100)],
+                                  [(2, 3000 + 100 * i) for i in range(12)]])
+def test_bf16_tile_launches_by_query_bounds(D, seqs):
+    """All sequences above 16 queries (the 32-row kernel alone), none, or both;
+    partitions of 64, 128 and 256 keys."""
+    b = make_batch(seqs, 8, 4, D, 16, seed=D + len(seqs))
+    check(run_attention(b, "bf16"), expected(b, "bf16"), "bf16")

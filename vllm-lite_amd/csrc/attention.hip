@@ -333,10 +333,18 @@ __device__ __forceinline__ SeqWork seq_work(int q, int c, const PlanLens& n, int
   return w;
 }
 
+// Shortest decode ranges: 128 tokens, doubled from half a compute unit's worth
+// of items on. Ranges of 64 (one block per wavefront) are no faster to read and
+// leave more partials to merge: 16 sequences of 100-900 tokens 35.3 us, at 128
+// 29.5, at 256 24.5; one of 8000 46.1, 31.9, 26.7; one of 500 21.4, 21.6, 22.6
+constexpr int kRangeMinLog2 = 7;
 constexpr int kRangeMaxLog2 = 11;
 constexpr int kRangeMax = 1 << kRangeMaxLog2;  // longest decode range the planner starts with
 constexpr int kItemsPerWg = 4;  // decode items aimed for per resident workgroup
-constexpr int kTileItemsPerWg = 4;  // split tile items aimed for per workgroup
+// Split tile items aimed for per workgroup. bf16: verify 64 x 5 722 us at 1, 711
+// at 2, 711 at 3, 729 at 4; 160 decodes at head_dim 64 52.5, 56, 63, 63; 8
+// verifies 160, 146, 156, 156
+constexpr int kTileItemsPerWg = 2;
 // fp32 ones have more work per key and pay their start and merge more often:
 // 24 decodes at head_dim 80 68 us at 4, 54 at 2, 48 at 1, with 2 chunks beside
 // them 79, 66 and 76
@@ -443,7 +451,7 @@ __device__ __forceinline__ int bucket_add(int* h, int key, int hot) {
 }
 
 // One workgroup. Chooses the bandwidth kernel's range length R (the smallest
-// power of two in 64..kRangeMax that leaves at most target_items (range, KV head)
+// power of two in 128..kRangeMax that leaves at most target_items (range, KV head)
 // items, i.e. a few per resident workgroup: longer ranges mean fewer split
 // partials to write and merge, shorter ones keep every CU busy) and the
 // multi-query partition length P (the smallest power of two from kPart0 that
@@ -459,7 +467,7 @@ __device__ __forceinline__ int bucket_add(int* h, int key, int hot) {
 template <bool kCached>
 __global__ void __launch_bounds__(kPlanThreads) plan_kernel(
     const int32_t* __restrict__ seq_lens, const int32_t* __restrict__ qsl, int S, int rep, int Hkv,
-    bool fast, bool tile, bool wide, int64_t cap_rows, int target_items, int tile_target,
+    bool fast, bool tile, bool wide, int64_t cap_rows, int target_items, int few_items, int tile_target,
     int chunk_target, int32_t* __restrict__ hdr, int32_t* __restrict__ gen_off,
     int32_t* __restrict__ tile_off, int32_t* __restrict__ nparts,
     int32_t* __restrict__ split_base, int32_t* __restrict__ wide_off,
@@ -481,7 +489,7 @@ __global__ void __launch_bounds__(kPlanThreads) plan_kernel(
   // 0. range length from the decode tokens and the target item count; the
   // same for the partition length of the splittable multi-query sequences
   // (at most kSplitMaxQ queries), counted in (KV head, 64-row block) units
-  PlanLens n = {kPart0Log2, kNoSplit, 6};
+  PlanLens n = {kPart0Log2, kNoSplit, kRangeMinLog2};
   bool lpt;  // 16-row items (or bf16 ones' last partitions) handed out longest first
   {
     unsigned long long v[3] = {0, 0, 0};
@@ -507,8 +515,17 @@ __global__ void __launch_bounds__(kPlanThreads) plan_kernel(
       while (l < to && keys * (unsigned long long)Hkv > (unsigned long long)max(target, 1) << l) ++l;
       return l;
     };
-    n.lr = fit(v[0], target_items, 6, kRangeMaxLog2);
-    n.lp = fit(v[1], tile_target, kPart0Log2, 20);
+    // ranges of 256 tokens, one burst of 4 blocks per wavefront, or 128 where
+    // that leaves fewer than half the compute units' worth of items
+    n.lr = fit(v[0], few_items, kRangeMinLog2, kRangeMinLog2 + 1);
+    n.lr = fit(v[0], target_items, n.lr, kRangeMaxLog2);
+    // bf16 partitions of 64 keys only while they leave at most an item per
+    // compute unit, then up to 256 before the items aimed for count: 20 decodes
+    // at head_dim 64 32.7 -> 21.5 us, 3 verifies of up to 2000 keys 35.4 ->
+    // 32.1. (fp32 items are longer: 24 decodes + 2 chunks at head_dim 80 77 us
+    // this way, 66 without.)
+    if (wide) n.lp = fit(v[1], 2 * few_items, kPart0Log2, kPart0Log2 + 2);
+    n.lp = fit(v[1], tile_target, n.lp, 20);
     if (v[2] > 0)
       n.p2 = (int)min((unsigned long long)kNoSplit,
                       max((unsigned long long)kChunkPart,
@@ -2986,7 +3003,7 @@ int do_plan(const Args& a, void* ws, size_t ws_bytes, hipStream_t st) {
   const int tile_target = wide ? kTileItemsPerWg * tile_grid() : kTileItemsPerWgF32 * tile_grid();
   auto* plan = a.S <= kPlanThreads * kPlanRegSeqs ? plan_kernel<true> : plan_kernel<false>;
   plan<<<1, kPlanThreads, 0, st>>>(a.seq_lens, a.qsl, a.S, a.H / a.Hkv, a.Hkv, fast, tile, wide,
-                                   L.cap_rows, target_items, tile_target, chunk_target,
+                                   L.cap_rows, target_items, vl_num_cus() / 2, tile_target, chunk_target,
                                    L.hdr, L.gen_off,
                                    L.tile_off, L.nparts, L.split_base, L.wide_off, L.cmb_seq,
                                    L.wide_seq, L.tail_seq, L.tail_off, L.desc, L.ml);
@@ -3036,21 +3053,23 @@ int launch_tile_d(const Args& a, const Layout& L, float sl2, hipStream_t st) {
   return VL_OK;
 }
 
-// The 16-row tile kernel always (short-query and fp32 items); for bf16 head
-// dims 64 and 128 also the 32-row kernel when a sequence may have more than
-// kSplitMaxQ queries.
+// The 16-row tile kernel (short-query and fp32 items); for bf16 head dims 64
+// and 128 also the 32-row kernel when a sequence may have more than
+// kSplitMaxQ queries, and that one alone when all have (the launch that finds
+// no item took 4.7 us of 219 for 12 ragged prefill chunks).
 template <typename T, typename TKV = T>
-int launch_tile(const Args& a, const Layout& L, float sl2, int max_q, hipStream_t st) {
+int launch_tile(const Args& a, const Layout& L, float sl2, int max_q, int min_q, hipStream_t st) {
   const bool wide = max_q <= 0 || max_q > kSplitMaxQ;
+  const bool narrow = min_q <= kSplitMaxQ;  // 0: unknown
   int rc = VL_OK;
   if constexpr (sizeof(T) == 2) {
     switch (a.D) {
       case 64:
-        rc = launch_tile_d<T, 64, 16>(a, L, sl2, st);
+        if (narrow) rc = launch_tile_d<T, 64, 16>(a, L, sl2, st);
         if (!rc && wide) rc = launch_tile_d<T, 64, 32>(a, L, sl2, st);
         return rc;
       case 128:
-        rc = launch_tile_d<T, 128, 16>(a, L, sl2, st);
+        if (narrow) rc = launch_tile_d<T, 128, 16>(a, L, sl2, st);
         if (!rc && wide) rc = launch_tile_d<T, 128, 32>(a, L, sl2, st);
         return rc;
       case 16: return launch_tile_d<float, 16, 16, T, T>(a, L, sl2, st);
@@ -3146,7 +3165,7 @@ int do_run(const Args& a, int max_q, int min_q, int max_ctx, void* ws, size_t ws
   const bool fast = one_type && fast_shape(a.dtype, a.H, a.Hkv, a.D, a.bs);
   if constexpr (!one_type) {
     if (tile_shape(a.dtype, a.D, a.bs)) {
-      const int rc = launch_tile<T, TKV>(a, L, sl2, max_q, st);
+      const int rc = launch_tile<T, TKV>(a, L, sl2, max_q, min_q, st);
       if (rc) return rc;
     }
   } else if (fast) {
@@ -3170,11 +3189,11 @@ int do_run(const Args& a, int max_q, int min_q, int max_ctx, void* ws, size_t ws
       VL_CHECK_LAUNCH();
     }
     if (!step_all && !(known && min_q == 1)) {
-      const int rc = launch_tile<T>(a, L, sl2, max_q, st);
+      const int rc = launch_tile<T>(a, L, sl2, max_q, min_q, st);
       if (rc) return rc;
     }
   } else if (tile_shape(a.dtype, a.D, a.bs)) {
-    int rc = launch_tile<T>(a, L, sl2, max_q, st);
+    int rc = launch_tile<T>(a, L, sl2, max_q, min_q, st);
     if (rc) return rc;
   }
   if (!fast && !tile_shape(a.dtype, a.D, a.bs)) {
@@ -3223,11 +3242,11 @@ extern "C" size_t vl_paged_attention_workspace_size(int num_seqs, int num_tokens
   int64_t parts = std::min<int64_t>(std::max<int64_t>(cdiv64(ctx, kPart0), 1), 64);
   // (and a split sequence's arrival counters, at most one row per query row)
   const int64_t rows_tile = parts > 1 ? split_tokens * H * (parts + 1) : 0;
-  // decode ranges: as short as 64 tokens for small batches, at most a few
+  // decode ranges: as short as 128 tokens for small batches, at most a few
   // items per resident workgroup (plus one short range per sequence) and at
   // most kRangeMax (2048) tokens long otherwise
   const int64_t rows_fast =
-      std::min<int64_t>(S * H * cdiv64(ctx, 64),
+      std::min<int64_t>(S * H * (cdiv64(ctx, 1 << kRangeMinLog2) + 1),
                         4 * kItemsPerWg * (int64_t)decode_grid() +
                             S * H * (cdiv64(ctx, kRangeMax) + 1));
   // split fp32 chunks: sum q H np <= 2 sum q H c / P2 (np >= 2 parts), with P2
