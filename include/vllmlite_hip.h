@@ -357,8 +357,8 @@ int vl_decode_attention_wo(float* parts, const float* query, int64_t query_strid
 
 /*
  * A copy of n int32 words by one kernel (no counterpart in the reference,
- * which has no device): src may be pinned host memory (hipHostMalloc), read
- * by the kernel over the bus. A step graph's host-to-device copy of its
+ * which has no device): src or dst may be pinned host memory (hipHostMalloc),
+ * read or written by the kernel over the bus. A step graph's host-to-device copy of its
  * staging record, as a memcpy node, costs ~12 us more per step than this
  * kernel node.
  */

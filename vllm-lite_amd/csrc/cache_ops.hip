@@ -232,8 +232,9 @@ extern "C" int vl_rope_and_cache(const float* qkv, int64_t qkv_stride, float* q_
   return VL_OK;
 }
 
-// One workgroup copies n int32 words; src may be pinned host memory, read
-// over the bus by the kernel itself (16-byte loads when both ends allow).
+// One workgroup copies n int32 words; src or dst may be pinned host memory, read
+// or written over the bus by the kernel itself (16 bytes at a time when both
+// ends allow).
 __global__ void __launch_bounds__(256) copy_words_kernel(int32_t* __restrict__ dst,
                                                          const int32_t* __restrict__ src,
                                                          int64_t n) {

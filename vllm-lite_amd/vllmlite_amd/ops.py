@@ -754,7 +754,7 @@ def decode_attention_wo(parts: torch.Tensor, query: torch.Tensor, key_cache: tor
 
 
 def copy_words(dst: torch.Tensor, src: torch.Tensor) -> None:
-    """dst[:] = src (int32, src may be pinned host memory) by one kernel
+    """dst[:] = src (int32, either may be pinned host memory) by one kernel
     (vl_copy_words)."""
     _need(dst.dtype == torch.int32 and src.dtype == torch.int32 and dst.is_contiguous() and
           src.is_contiguous() and dst.numel() == src.numel(), "int32 tensors of one size required")
