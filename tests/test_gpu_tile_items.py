@@ -109,8 +109,7 @@ def test_widened_head_dims_over_an_fp8_cache(D):
                                   [(1, 255 + 64 * i) for i in range(24)]])
 @pytest.mark.parametrize("small_ws", [False, True])
 def test_short_decode_batches_of_the_bandwidth_kernel(seqs, small_ws):
-    """Few items: ranges of 128 tokens, doubled to 256 from half a compute
-    unit's worth of items on; contexts around a range's end."""
+    """Few items, the shortest ranges; contexts around a range's end."""
     b = make_batch(seqs, 32, 8, 128, 16, seed=len(seqs))
     ws = ops().lib().vl_paged_attention_min_workspace(len(seqs)) if small_ws else None
     check(run_attention(b, "bf16", ws_bytes=ws), expected(b, "bf16"), "bf16")
@@ -120,7 +119,6 @@ def test_short_decode_batches_of_the_bandwidth_kernel(seqs, small_ws):
 @pytest.mark.parametrize("seqs", [[(17, 17), (400, 900)], [(16, 900), (17, 300)], [(5, 100)],
                                   [(2, 3000 + 100 * i) for i in range(12)]])
 def test_bf16_tile_launches_by_query_bounds(D, seqs):
-    """All sequences above 16 queries (the 32-row kernel alone), none, or both;
-    partitions of 64, 128 and 256 keys."""
+    """All sequences above 16 queries (the 32-row kernel alone), none, or both."""
     b = make_batch(seqs, 8, 4, D, 16, seed=D + len(seqs))
     check(run_attention(b, "bf16"), expected(b, "bf16"), "bf16")

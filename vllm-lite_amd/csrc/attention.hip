@@ -333,11 +333,12 @@ __device__ __forceinline__ SeqWork seq_work(int q, int c, const PlanLens& n, int
   return w;
 }
 
-// Shortest decode ranges: 128 tokens, doubled from half a compute unit's worth
-// of items on. Ranges of 64 (one block per wavefront) are no faster to read and
-// leave more partials to merge: 16 sequences of 100-900 tokens 35.3 us, at 128
-// 29.5, at 256 24.5; one of 8000 46.1, 31.9, 26.7; one of 500 21.4, 21.6, 22.6
-constexpr int kRangeMinLog2 = 7;
+// Shortest decode ranges: 64 tokens, one block per wavefront. Longer ones are
+// faster for small batches (16 sequences of 100-900 tokens 35.3 us, at 128 29.5,
+// at 256 24.5) but further from the 64-bit result (4 sequences 1.95e-3, at 128
+// 2.09e-3: the weights are rounded to bf16 relative to a range's maximum, which
+// is exact, and fewer of them are maxima)
+constexpr int kRangeMinLog2 = 6;
 constexpr int kRangeMaxLog2 = 11;
 constexpr int kRangeMax = 1 << kRangeMaxLog2;  // longest decode range the planner starts with
 constexpr int kItemsPerWg = 4;  // decode items aimed for per resident workgroup
@@ -451,7 +452,7 @@ __device__ __forceinline__ int bucket_add(int* h, int key, int hot) {
 }
 
 // One workgroup. Chooses the bandwidth kernel's range length R (the smallest
-// power of two in 128..kRangeMax that leaves at most target_items (range, KV head)
+// power of two in 64..kRangeMax that leaves at most target_items (range, KV head)
 // items, i.e. a few per resident workgroup: longer ranges mean fewer split
 // partials to write and merge, shorter ones keep every CU busy) and the
 // multi-query partition length P (the smallest power of two from kPart0 that
@@ -467,7 +468,7 @@ __device__ __forceinline__ int bucket_add(int* h, int key, int hot) {
 template <bool kCached>
 __global__ void __launch_bounds__(kPlanThreads) plan_kernel(
     const int32_t* __restrict__ seq_lens, const int32_t* __restrict__ qsl, int S, int rep, int Hkv,
-    bool fast, bool tile, bool wide, int64_t cap_rows, int target_items, int few_items, int tile_target,
+    bool fast, bool tile, bool wide, int64_t cap_rows, int target_items, int tile_target,
     int chunk_target, int32_t* __restrict__ hdr, int32_t* __restrict__ gen_off,
     int32_t* __restrict__ tile_off, int32_t* __restrict__ nparts,
     int32_t* __restrict__ split_base, int32_t* __restrict__ wide_off,
@@ -515,17 +516,8 @@ __global__ void __launch_bounds__(kPlanThreads) plan_kernel(
       while (l < to && keys * (unsigned long long)Hkv > (unsigned long long)max(target, 1) << l) ++l;
       return l;
     };
-    // ranges of 256 tokens, one burst of 4 blocks per wavefront, or 128 where
-    // that leaves fewer than half the compute units' worth of items
-    n.lr = fit(v[0], few_items, kRangeMinLog2, kRangeMinLog2 + 1);
-    n.lr = fit(v[0], target_items, n.lr, kRangeMaxLog2);
-    // bf16 partitions of 64 keys only while they leave at most an item per
-    // compute unit, then up to 256 before the items aimed for count: 20 decodes
-    // at head_dim 64 32.7 -> 21.5 us, 3 verifies of up to 2000 keys 35.4 ->
-    // 32.1. (fp32 items are longer: 24 decodes + 2 chunks at head_dim 80 77 us
-    // this way, 66 without.)
-    if (wide) n.lp = fit(v[1], 2 * few_items, kPart0Log2, kPart0Log2 + 2);
-    n.lp = fit(v[1], tile_target, n.lp, 20);
+    n.lr = fit(v[0], target_items, kRangeMinLog2, kRangeMaxLog2);
+    n.lp = fit(v[1], tile_target, kPart0Log2, 20);
     if (v[2] > 0)
       n.p2 = (int)min((unsigned long long)kNoSplit,
                       max((unsigned long long)kChunkPart,
@@ -3003,7 +2995,7 @@ int do_plan(const Args& a, void* ws, size_t ws_bytes, hipStream_t st) {
   const int tile_target = wide ? kTileItemsPerWg * tile_grid() : kTileItemsPerWgF32 * tile_grid();
   auto* plan = a.S <= kPlanThreads * kPlanRegSeqs ? plan_kernel<true> : plan_kernel<false>;
   plan<<<1, kPlanThreads, 0, st>>>(a.seq_lens, a.qsl, a.S, a.H / a.Hkv, a.Hkv, fast, tile, wide,
-                                   L.cap_rows, target_items, vl_num_cus() / 2, tile_target, chunk_target,
+                                   L.cap_rows, target_items, tile_target, chunk_target,
                                    L.hdr, L.gen_off,
                                    L.tile_off, L.nparts, L.split_base, L.wide_off, L.cmb_seq,
                                    L.wide_seq, L.tail_seq, L.tail_off, L.desc, L.ml);
@@ -3242,11 +3234,11 @@ extern "C" size_t vl_paged_attention_workspace_size(int num_seqs, int num_tokens
   int64_t parts = std::min<int64_t>(std::max<int64_t>(cdiv64(ctx, kPart0), 1), 64);
   // (and a split sequence's arrival counters, at most one row per query row)
   const int64_t rows_tile = parts > 1 ? split_tokens * H * (parts + 1) : 0;
-  // decode ranges: as short as 128 tokens for small batches, at most a few
+  // decode ranges: as short as 64 tokens for small batches, at most a few
   // items per resident workgroup (plus one short range per sequence) and at
   // most kRangeMax (2048) tokens long otherwise
   const int64_t rows_fast =
-      std::min<int64_t>(S * H * (cdiv64(ctx, 1 << kRangeMinLog2) + 1),
+      std::min<int64_t>(S * H * cdiv64(ctx, 1 << kRangeMinLog2),
                         4 * kItemsPerWg * (int64_t)decode_grid() +
                             S * H * (cdiv64(ctx, kRangeMax) + 1));
   // split fp32 chunks: sum q H np <= 2 sum q H c / P2 (np >= 2 parts), with P2

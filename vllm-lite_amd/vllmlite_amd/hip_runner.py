@@ -64,13 +64,14 @@ from .runner import ModelRunner
 # of the default model: 1747 us, by the fused kernels 1813)
 FUSED_ROWS_MAX = 1024
 # decode steps with wo inside the attention launch (one partial row per KV
-# head, summed again by every workgroup of gate|up): up to this many rows and
-# this d_model. The partial rows and the wo columns an attention workgroup
-# multiplies by grow with both: d_model 384, 8 heads over 4 or 8: 16 rows 190
-# and 198 us per step against 197 and 199 with wo in a launch of its own, 32 rows
-# 229 and 253 against 223 and 231; d_model 512 (6 layers, d_ff 2048, 8 over 8):
-# 4 rows 245 against 216, 16 rows 264 against 235, 32 rows 376 against 346
-FUSED_WO_ROWS = 16
+# head and row, summed again by every workgroup of gate|up): up to this many
+# partial rows, and up to this d_model (the wo columns an attention workgroup
+# multiplies by). Per step, fused against wo in a launch of its own, rows x KV
+# heads: d_model 384, 16 x 4 190 and 197 us, 16 x 8 198 and 199, 32 x 4 229 and
+# 223, 32 x 8 253 and 231; d_model 256, 16 x 2 177 and 200, 32 x 2 206 and 213,
+# 16 x 8 184 and 182, 32 x 4 208 and 207; d_model 512 (d_ff 2048), 16 x 4 238 and
+# 229, 4 x 8 245 and 216, 32 x 8 376 and 346
+FUSED_WO_PARTS = 64
 FUSED_WO_D_MODEL = 384
 # execute() writes up to this many logits to the pinned host buffer by a kernel
 # (one workgroup), more by a copy: 16 x 261 186.5 against 193 us per step, 16 x
@@ -692,7 +693,7 @@ class HipRunner(ModelRunner):
         launch (one partial row per KV head) and the residual add in gate|up's
         prologue: four launches per layer."""
         W, Tb, Rb = self.w, s.Tb, s.Rb
-        if s.decode and self._fused_wo and Tb <= FUSED_WO_ROWS:
+        if s.decode and self._fused_wo and Tb * self.Hkv <= FUSED_WO_PARTS:
             self._forward_decode_wo(s, x, q, act, lidx, qsl, lens, bt, ids_host, rec_host)
             return
         pos = self._meta[s.pos:s.pos + Tb]
