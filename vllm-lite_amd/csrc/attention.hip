@@ -342,10 +342,10 @@ constexpr int kRangeMinLog2 = 6;
 constexpr int kRangeMaxLog2 = 11;
 constexpr int kRangeMax = 1 << kRangeMaxLog2;  // longest decode range the planner starts with
 constexpr int kItemsPerWg = 4;  // decode items aimed for per resident workgroup
-// Split tile items aimed for per workgroup. bf16: verify 64 x 5 722 us at 1, 711
-// at 2, 711 at 3, 729 at 4; 160 decodes at head_dim 64 52.5, 56, 63, 63; 8
-// verifies 160, 146, 156, 156
-constexpr int kTileItemsPerWg = 2;
+// Split tile items aimed for per workgroup. bf16: 160 decodes at head_dim 64 run
+// 57 us at 2 and 64 at 4, but verify 64 x 5 over six draws of contexts 710, 788,
+// 750, 814, 703, 871 at 2 and 727, 764, 730, 793, 721, 839 at 4
+constexpr int kTileItemsPerWg = 4;
 // fp32 ones have more work per key and pay their start and merge more often:
 // 24 decodes at head_dim 80 68 us at 4, 54 at 2, 48 at 1, with 2 chunks beside
 // them 79, 66 and 76
