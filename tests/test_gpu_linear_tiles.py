@@ -18,13 +18,29 @@ def _dev(a):
     return torch.from_numpy(np.ascontiguousarray(a)).cuda()
 
 
+def _rows_per_workgroup(rows, n):
+    """What the dispatch takes for this many rows and columns (linear.hip:
+    takes_tiles, launch_tiles): 64- or 32-row workgroups of
+    linear_tile_kernel, or 0 (linear_rows_kernel)."""
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    cb = -(-(-(-n // 16)) // 4)
+    if cb * -(-rows // 32) < cus:
+        return 0
+    return 64 if cb * -(-rows // 64) >= 2 * cus else 32
+
+
 # 32- and 64-row workgroups, a last row block and a last column block that are
 # not full, K below a chunk of 64, a multiple of it and not
-@pytest.mark.parametrize("rows,k,n,mode", [(1400, 1024, 384, "accumulate"), (1000, 496, 1100, "store"),
-                                           (1030, 384, 1152, "store"), (700, 64, 1030, "swiglu"),
-                                           (260, 512, 2048, "swiglu"), (2050, 16, 520, "store")])
+@pytest.mark.parametrize("rows,k,n,mode,wg_rows",
+                         [(1400, 1024, 384, "accumulate", 32), (1000, 496, 1100, "store", 32),
+                          (1030, 384, 1152, "store", 32), (700, 64, 1030, "swiglu", 32),
+                          (260, 512, 2048, "swiglu", 32), (2050, 16, 520, "store", 32),
+                          (1024, 512, 2048, "swiglu", 64), (1000, 400, 2041, "swiglu", 64),
+                          (2050, 16, 1030, "store", 64), (2050, 336, 1100, "store", 64),
+                          (4111, 1024, 512, "accumulate", 64)])
 @pytest.mark.parametrize("norm", [False, True])
-def test_many_rows_over_tiled_weights(rows, k, n, mode, norm):
+def test_many_rows_over_tiled_weights(rows, k, n, mode, wg_rows, norm):
+    assert _rows_per_workgroup(rows, n) == wg_rows
     o = _ops()
     rng = np.random.default_rng(rows + k + norm)
     halves = 2 if mode == "swiglu" else 1
@@ -43,9 +59,11 @@ def test_many_rows_over_tiled_weights(rows, k, n, mode, norm):
     _close(out.cpu().numpy(), want)
 
 
-@pytest.mark.parametrize("rows", [1, 16, 33, 1100])
+@pytest.mark.parametrize("rows", [1, 16, 33, 1100, 4111])
 @pytest.mark.parametrize("k,n", [(16, 512), (1040, 40), (2048, 512)])
 def test_deep_projection(rows, k, n):
+    assert _rows_per_workgroup(rows, n) == (0 if rows < 1100 or n < 512 else
+                                            32 if rows == 1100 else 64)
     o = _ops()
     rng = np.random.default_rng(rows + k)
     x = rng.standard_normal((rows, k)).astype(np.float32)
@@ -66,28 +84,31 @@ def test_deep_projection(rows, k, n):
 
 @pytest.mark.parametrize("layout", ["token", "head"])
 @pytest.mark.parametrize("cache", [torch.float32, torch.bfloat16])
-def test_many_rows_qkv_equals_projection_then_rope(layout, cache):
+@pytest.mark.parametrize("rows,wg_rows", [(1000, 32), (2741, 64)])
+def test_many_rows_qkv_equals_projection_then_rope(layout, cache, rows, wg_rows):
     """Rows gathered by index with placeholders, copied to x_out, the record
     copied too: the same bits as the projection of the gathered rows followed
     by vl_rope_and_cache."""
     o = _ops()
-    H, Hkv, D, k, rows = 8, 4, 48, 384, 1000
+    H, Hkv, D, k = 8, 4, 48, 384
     n = (H + 2 * Hkv) * D
+    assert _rows_per_workgroup(rows, n) == wg_rows
+    blocks = -(-rows // 16)
     rng = np.random.default_rng(3)
     table = _dev(rng.standard_normal((261, k)).astype(np.float32))
     prev = _dev(rng.integers(0, 261, 12).astype(np.int32))
     ids_np = rng.integers(0, 261, rows).astype(np.int32)
-    ids_np[[0, 500, 999]] = [-1, -12, -13]  # -13: past num_prev -> id 0
+    ids_np[[0, 500, rows - 1]] = [-1, -12, -13]  # -13: past num_prev -> id 0
     ids = _dev(ids_np)
     w = o.tile16(_dev((0.05 * rng.standard_normal((k, n))).astype(np.float32)))
     g = _dev((1.0 + 0.1 * rng.standard_normal(k)).astype(np.float32))
     pos = _dev(rng.integers(0, 64, rows).astype(np.int32))
-    slots = rng.permutation(1008)[:rows].astype(np.int32)
+    slots = rng.permutation(16 * blocks)[:rows].astype(np.int32)
     slots[::7] = -1
     slot = _dev(slots)
     ang = rng.standard_normal((64, D // 2)).astype(np.float32)
     cos, sin = _dev(np.cos(ang)), _dev(np.sin(ang))
-    shape = (63, Hkv, 16, D) if layout == "head" else (1008, Hkv, D)
+    shape = (blocks, Hkv, 16, D) if layout == "head" else (16 * blocks, Hkv, D)
     kc1, vc1, kc2, vc2 = (torch.zeros(shape, device="cuda", dtype=cache) for _ in range(4))
     q1, q2 = torch.empty((rows, H, D), device="cuda"), torch.empty((rows, H * D), device="cuda")
     x_out = torch.full((rows, k), float("nan"), device="cuda")
@@ -124,3 +145,34 @@ def test_deeper_models_match_the_oracle_runner(shape):
     for (g, dec), (w, _) in zip(got, want):
         scale = np.abs(w).max(axis=-1, keepdims=True)
         assert np.all(np.abs(g - w) <= 2e-4 * scale), f"decode step {dec}"
+
+
+@pytest.mark.parametrize("lens,bucket", [((211, 300, 169), 1024), ((120, 99), 256)])
+def test_long_prompts_through_the_runner(lens, bucket):
+    """Prefill steps of a model with d_ff 2048 large enough that its
+    projections take linear_tile_kernel (layer 0's gather, residual copy and
+    record among them), with rows past the step's tokens in the bucket: the
+    logits of that step and of the decodes after it, and every layer's cached
+    K and V, against the oracle runner, within 2e-4 of the largest."""
+    from oracle.runner import NumpyRunner
+    from vllmlite_amd.hip_runner import HipRunner
+    cfg = small_cfg(layers=2)
+    for f, v in dict(n_heads=8, n_kv_heads=8, d_model=512, d_ff=2048).items():
+        setattr(cfg.model, f, v)
+    assert bucket // 2 < sum(n + 1 for n in lens) < bucket
+    assert _rows_per_workgroup(bucket, 2048) == (64 if bucket == 1024 else 32)
+    rng = np.random.default_rng(bucket)
+    prompts = ["".join(chr(c) for c in rng.integers(32, 127, n)) for n in lens]
+    runners = []
+
+    def made(cls):
+        return lambda m, c: runners.append(cls(m, c)) or runners[-1]
+
+    got = _logit_trace(made(HipRunner), cfg, prompts, 3)
+    want = _logit_trace(made(NumpyRunner), cfg, prompts, 3)
+    assert len(got) == len(want)
+    for (g, dec), (w, _) in zip(got, want):
+        assert np.all(np.abs(g - w) <= 2e-4 * np.abs(w).max(axis=-1, keepdims=True)), dec
+    for name in ("cache_k", "cache_v"):
+        g, w = getattr(runners[0], name).cpu().numpy(), getattr(runners[1], name)
+        assert np.abs(g - w).max() <= 2e-4 * np.abs(w).max(), name
