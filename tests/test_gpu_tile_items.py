@@ -122,3 +122,22 @@ def test_bf16_tile_launches_by_query_bounds(D, seqs):
     """All sequences above 16 queries (the 32-row kernel alone), none, or both."""
     b = make_batch(seqs, 8, 4, D, 16, seed=D + len(seqs))
     check(run_attention(b, "bf16"), expected(b, "bf16"), "bf16")
+
+
+@pytest.mark.parametrize("H,Hkv,D", [(2, 1, 64), (4, 2, 80)])
+def test_split_chunk_with_rows_before_the_first_position(H, Hkv, D):
+    """More queries than context: queries at negative positions see no key, and
+    their rows are written as zeros also where the chunk's context is cut (the
+    first row blocks then reach no part). The others match the oracle."""
+    o = ops()
+    q_len, ctx = 700, 300
+    b = make_batch([(q_len, ctx)], H, Hkv, D, 16, seed=D)
+    q = dev(b["q"])
+    out = torch.full_like(q, float("nan"))
+    ws = o.AttentionWorkspace().get(o.paged_attention_workspace_size(1, q_len, H, D, ctx))
+    o.paged_attention(out, q, dev(b["k_cache"]), dev(b["v_cache"]), dev(b["block_tables"]),
+                      dev(b["seq_lens"]), dev(b["qsl"]), b["scale"], 16, ws, max_query_len=q_len)
+    got = to_np(out)
+    assert np.array_equal(got[:q_len - ctx], np.zeros_like(got[:q_len - ctx]))
+    seen = dict(b, q=b["q"][q_len - ctx:], qsl=np.array([0, ctx], np.int32))
+    check(got[q_len - ctx:], oracle_attention(seen), "f32")

@@ -1264,11 +1264,13 @@ __device__ __forceinline__ void tile_body(TileLds<T, D, RW>& lds, int it, int pa
     const int blk_last = min(nrows - 1, rbase + kRows - 1);
     const int kend_wg = min(kend, ctx - q_len + blk_last / rep + 1);
     // the partitions that reach the row block's keys: of a split chunk's (fp32)
-    // row block, those past its last row's position have no work
+    // row block, those past its last row's position have no work. The first one
+    // always has: rows that see no key (more queries than context) get their
+    // zeros from it
     int ne = np;
     if constexpr (!kBf16) {
       if (np > 1 && q_len > kSplitMaxQ) {
-        ne = cdiv(ctx - q_len + blk_last / rep + 1, P);
+        ne = max(1, cdiv(ctx - q_len + blk_last / rep + 1, P));
         if (part >= ne) return;
       }
     }
