@@ -110,7 +110,8 @@ size_t vl_paged_attention_min_workspace(int num_seqs);
  * 0..ceil(seq_lens[i]/block_size)). Query j of a sequence with q_len tokens
  * sits at position seq_lens[i] - q_len + j and attends keys 0..position
  * (causal; a single query sees the whole context; a query at a negative
- * position sees none and its output is zero). Head h reads KV head
+ * position sees none and its output is zero; the outputs of a sequence with
+ * seq_lens 0 may be left unwritten). Head h reads KV head
  * h / (num_heads / num_kv_heads). The caches are kv_layout. out [num_tokens,
  * num_heads, head_dim], contiguous, dtype of the query. Accumulation is fp32.
  * Launch hints, each 0 when unknown: max_query_len and min_query_len bound

@@ -141,3 +141,29 @@ def test_split_chunk_with_rows_before_the_first_position(H, Hkv, D):
     assert np.array_equal(got[:q_len - ctx], np.zeros_like(got[:q_len - ctx]))
     seen = dict(b, q=b["q"][q_len - ctx:], qsl=np.array([0, ctx], np.int32))
     check(got[q_len - ctx:], oracle_attention(seen), "f32")
+
+
+@pytest.mark.parametrize("dtype,D", [("f32", 80), ("bf16", 96), ("bf16", 32), ("f32", 48)])
+@pytest.mark.parametrize("seqs", [[(2, 0), (40, 300), (1, 0), (5, 700), (40, 0), (1, 1)], [(3, 0)],
+                                  [(30, 0), (1, 0)]])
+def test_queries_without_context_are_written_as_zeros(dtype, D, seqs):
+    """At the head dims whose items run fp32 products, as the generic kernel
+    does at its own, beside other sequences and alone."""
+    o = ops()
+    tdt = torch.float32 if dtype == "f32" else torch.bfloat16
+    b = make_batch(seqs, 4, 2, D, 16, seed=D)
+    q = dev(b["q"], tdt)
+    out = torch.full_like(q, float("nan"))
+    S, T = len(seqs), q.shape[0]
+    ws = o.AttentionWorkspace().get(o.paged_attention_workspace_size(S, T, 4, D, 700))
+    o.paged_attention(out, q, dev(b["k_cache"], tdt), dev(b["v_cache"], tdt),
+                      dev(b["block_tables"]), dev(b["seq_lens"]), dev(b["qsl"]), b["scale"], 16, ws)
+    got = to_np(out)
+    for i, (q_len, ctx) in enumerate(seqs):
+        rows = slice(b["qsl"][i], b["qsl"][i + 1])
+        if ctx == 0:
+            assert np.array_equal(got[rows], np.zeros_like(got[rows]))
+        else:
+            one = dict(b, q=b["q"][rows], qsl=np.array([0, q_len], np.int32),
+                       tables=b["tables"][i:i + 1], seq_lens=b["seq_lens"][i:i + 1])
+            check(got[rows], expected(one, dtype), dtype)

@@ -308,7 +308,9 @@ __device__ __forceinline__ int cdiv_pow2(int a, int l) { return (int)(((int64_t)
 __device__ __forceinline__ SeqWork seq_work(int q, int c, const PlanLens& n, int rep, int Hkv,
                                             bool fast, bool tile, bool wide) {
   SeqWork w;
-  const bool live = q > 0 && c > 0;
+  // a sequence without context has no work, except fp32 tile items: they write
+  // its queries' zeros, as the generic kernel does for its head dims
+  const bool live = q > 0 && (c > 0 || !wide);
   const bool bw = is_bw(q, c, fast);
   const bool tl = !bw && tile && live;
   if (bw) {
@@ -522,7 +524,7 @@ __global__ void __launch_bounds__(kPlanThreads) plan_kernel(
       n.p2 = (int)min((unsigned long long)kNoSplit,
                       max((unsigned long long)kChunkPart,
                           v[2] * (unsigned long long)Hkv / max(chunk_target, 1)));
-    lpt = wide ? v[1] > 0 : v[1] + v[2] > 0;
+    lpt = wide ? v[1] > 0 : tile;
   }
   // 1. double P and R until the split partials fit (every thread holds the
   // same sums, so all take the same branch)
@@ -572,7 +574,8 @@ __global__ void __launch_bounds__(kPlanThreads) plan_kernel(
                          : q > kSplitMaxQ && w.np > 1 ? chunk_part_len(c, w.np)
                          : q > kSplitMaxQ             ? c
                                                       : min(c, P);
-    return kTailBuckets - 2 - (int)min<int64_t>(kTailBuckets - 2, cdiv64(last, kTileKeys) - 1);
+    return kTailBuckets - 2 -
+           (int)min<int64_t>(kTailBuckets - 2, max<int64_t>(cdiv64(last, kTileKeys), 1) - 1);
   };
   int64_t f = 0, g = 0, r = 0, x = 0, xs = 0, tl = 0, wd = 0, cm = 0;
   ch.each(qsl, seq_lens, [&](int, int q, int c) {
