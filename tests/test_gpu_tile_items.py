@@ -167,3 +167,14 @@ def test_queries_without_context_are_written_as_zeros(dtype, D, seqs):
             one = dict(b, q=b["q"][rows], qsl=np.array([0, q_len], np.int32),
                        tables=b["tables"][i:i + 1], seq_lens=b["seq_lens"][i:i + 1])
             check(got[rows], expected(one, dtype), dtype)
+
+
+@pytest.mark.parametrize("scale", [0.0, -0.11])
+@pytest.mark.parametrize("dtype,D", [("f32", 80), ("f32", 48), ("bf16", 112), ("bf16", 32)])
+def test_fp32_tiles_take_any_sign_of_scale(dtype, D, scale):
+    """A scale of 0 (every visible key weighs the same) and a negative one: a
+    masked score is -inf whatever the scale. Narrow items, several row blocks,
+    a cut context."""
+    seqs = [(37, 37), (70, 300), (1, 700), (3, 90), (17, 500)]
+    b = dict(make_batch(seqs, 4, 2, D, 16, seed=D), scale=scale)
+    check(run_attention(b, dtype), expected(b, dtype), dtype)

@@ -1295,8 +1295,16 @@ __device__ __forceinline__ void tile_body(TileLds<T, D, RW>& lds, int it, int pa
     const int32_t* table = bt + (int64_t)i * bt_stride;
     const int64_t kv_off = (int64_t)kvh * head_stride;
 
-    // Q^T operand of the QK^T product, kept in registers for the whole item
+    // Q^T operand of the QK^T product, kept in registers for the whole item.
+    // The fp32 path takes any scale, as the generic kernel does: its sign goes
+    // into q (exactly; a scale of 0 makes q 0), so that a masked score, -inf
+    // times what is left of it, stays -inf and the largest score the maximum.
     typename std::conditional<kBf16, bf16x8_t, float>::type qop[kKS];
+    float q_sign = 1.f;
+    if constexpr (!kBf16) {
+      q_sign = scale_log2 < 0.f ? -1.f : scale_log2 == 0.f ? 0.f : 1.f;
+      scale_log2 = scale_log2 == 0.f ? 1.f : fabsf(scale_log2);
+    }
     {
       const TIO* qrow = query + (int64_t)tok * q_stride + (int64_t)head * D;
 #pragma unroll
@@ -1312,7 +1320,7 @@ __device__ __forceinline__ void tile_body(TileLds<T, D, RW>& lds, int it, int pa
             const f32x4_t w =
                 row_ok ? load4<kLoose>(qrow + 4 * s + 4 * grp) : (f32x4_t){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int e = 0; e < 4; ++e) qop[s + e] = w[e];
+            for (int e = 0; e < 4; ++e) qop[s + e] = w[e] * q_sign;
           }
         }
       }
