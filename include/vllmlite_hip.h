@@ -114,6 +114,11 @@ size_t vl_paged_attention_min_workspace(int num_seqs);
  * seq_lens 0 may be left unwritten). Head h reads KV head
  * h / (num_heads / num_kv_heads). The caches are kv_layout. out [num_tokens,
  * num_heads, head_dim], contiguous, dtype of the query. Accumulation is fp32.
+ * An infinite or NaN element of a cached V row makes that element of the
+ * outputs of the queries that see it infinite or NaN; with a power-of-two
+ * block size, at head_dim 64 and 128 and (fp32 queries) 16, 32 and 48, also
+ * that of up to 63 queries of the sequence just before them (a masked key
+ * enters their sums with weight 0).
  * Launch hints, each 0 when unknown: max_query_len and min_query_len bound
  * the query count of the sequences with at least one query, max_context_len
  * bounds seq_lens. With max_query_len 1 and max_context_len <= 2048, head_dim

@@ -178,3 +178,31 @@ def test_fp32_tiles_take_any_sign_of_scale(dtype, D, scale):
     seqs = [(37, 37), (70, 300), (1, 700), (3, 90), (17, 500)]
     b = dict(make_batch(seqs, 4, 2, D, 16, seed=D), scale=scale)
     check(run_attention(b, dtype), expected(b, dtype), dtype)
+
+
+@pytest.mark.parametrize("value", [np.inf, -np.inf, np.nan])
+@pytest.mark.parametrize("dtype,D", [("f32", 80), ("f32", 96), ("f32", 112), ("bf16", 16),
+                                     ("bf16", 48), ("bf16", 80)])
+def test_a_value_row_that_is_not_finite_reaches_only_queries_that_see_it(dtype, D, value):
+    """One element of a V row that later queries of the chunk see and earlier
+    ones do not, at the head dims without an alignment rule: the earlier rows
+    are what they are with the element finite, the others are not finite at
+    that dim of that KV head, and every other element is unchanged. Chunks of
+    several row blocks, of one, of at most 16 rows, a cut context; the element
+    in a full tile, on the diagonal and in the last tile's last key."""
+    H, Hkv, bs, d0, g0 = 4, 2, 16, D - 3, 1
+    seqs = [(130, 130), (40, 321), (3, 90), (8, 64), (300, 1100)]
+    at = [70, 300, 88, 63, 900]  # the key whose V element is not finite
+    b = make_batch(seqs, H, Hkv, D, bs, seed=D)
+    want = expected(b, dtype)
+    v = b["v_cache"].copy()
+    sees = np.zeros(want.shape[0], bool)
+    for i, ((q_len, ctx), key) in enumerate(zip(seqs, at)):
+        v[b["tables"][i][key // bs] * bs + key % bs, g0, d0] = value
+        sees[b["qsl"][i]:b["qsl"][i + 1]] = ctx - q_len + np.arange(q_len) >= key
+    assert sees.any() and not sees.all()
+    got = run_attention(dict(b, v_cache=v), dtype)
+    heads = slice(g0 * (H // Hkv), (g0 + 1) * (H // Hkv))
+    assert not np.isfinite(got[sees, heads, d0]).any()
+    got[sees, heads, d0] = want[sees, heads, d0]
+    check(got, want, dtype)

@@ -1794,6 +1794,58 @@ __device__ __forceinline__ void tile_body(TileLds<T, D, RW>& lds, int it, int pa
       if (ntile > 0) prefetch(kbeg, pk, pv);
       for (int ti = 0; ti < ntile; ++ti) tile_step(ti, 1, pk, pv);
     }
+    if constexpr (kLoose) {
+      // A masked key of a tile enters the PV product with weight 0, which times an
+      // infinite or NaN element of its V row is NaN. The head dims without an
+      // alignment rule keep what their generic kernel gave (a V row reaches only
+      // the queries that see its key): a wavefront of an item with masked keys
+      // that ends on a NaN computes its rows again, key by key. (Looking for
+      // such elements as a tile is staged cost 2-5 % of a mixed batch.)
+      bool nan = false;
+      if (kend_wg - 1 > ctx - q_len + rbase / rep) {  // uniform
+#pragma unroll
+        for (int u = 0; u < kDT; ++u)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) nan |= acc[u][r] != acc[u][r];
+      }
+      if (__any(nan)) {
+        // the keys its rows see, straight from the cache: a lane sums its
+        // operands' dims of the score, the row's 4 lanes add theirs, and each
+        // takes its dims of V (those of each4)
+        int grp4 = 4 * grp;
+        asm volatile("" : "+v"(grp4));  // nothing of this is kept across items
+        m_run = -__builtin_inff(), l_part = 0.f;
+#pragma unroll
+        for (int u = 0; u < kDT; ++u) acc[u] = (AccT){0.f, 0.f, 0.f, 0.f};
+        for (int key = kbeg; key < kend_wave; ++key) {
+          if (narrow && (key / 16) % 4 != wave) continue;  // another wavefront's key
+          const int64_t off = row_of(key);
+          float s = 0.f;
+#pragma unroll
+          for (int k = 0; k < kKS; ++k)
+            s = fmaf(qop[k], Elem<TKV>::load(kc + off, 16 * (k / 4) + grp4 + k % 4), s);
+          s += __shfl_xor(s, 16, 64);
+          s += __shfl_xor(s, 32, 64);
+          if (key > qpos) continue;
+          s *= scale_log2;
+          const float m_new = fmaxf(m_run, s);
+          const float ref = m_new == -__builtin_inff() ? 0.f : m_new;
+          const float alpha = exp2_fast(m_run - ref), p = exp2_fast(s - ref);
+          m_run = m_new;
+          l_part = fmaf(l_part, alpha, grp == 0 ? p : 0.f);
+#pragma unroll
+          for (int u = 0; u < kDT; ++u)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+              const int m = grp4 + r;
+              const int d = u < 4 * kQuads               ? 64 * (u / 4) + 4 * m + u % 4
+                            : u < 4 * kQuads + 2 * kPair ? 64 * kQuads + 2 * m + u % 2
+                                                         : 16 * u + m;
+              acc[u][r] = fmaf(p, Elem<TKV>::load(vc + off, d), acc[u][r] * alpha);
+            }
+        }
+      }
+    }
     if (!kBf16 && narrow) {
       // wavefront 0 takes the others' results, lane by lane, and writes
       if constexpr (!kBf16) {
