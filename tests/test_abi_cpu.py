@@ -51,6 +51,24 @@ def test_no_compute_without_gpu_needed_for_queries():
     assert lib.vl_abi_version() == 13
 
 
+def test_workspace_sizes_follow_what_the_plan_can_use():
+    """The recommended size for a 256-sequence decode batch, a 64 x 5 verify and
+    the default model's 2048-row runner buffers, in bytes; the cut of fp32
+    chunks over the context once added up to 105 MB to each."""
+    from vllmlite_amd.build import LIB_PATH
+    lib = ctypes.CDLL(LIB_PATH)
+    size = lib.vl_paged_attention_workspace_size
+    size.restype = ctypes.c_size_t
+    assert size(256, 256, 32, 128, 8192) <= 204e6
+    assert size(64, 320, 32, 128, 32768) <= 206e6
+    assert size(2048, 2048, 8, 64, 2112) <= 157e6
+    # few rows: every partition of 64 tokens fits, up to 8192 tokens
+    for rows, H, D, ctx in ((1, 4, 64, 8192), (4, 32, 128, 900), (5, 8, 80, 2000)):
+        fixed = lib.vl_paged_attention_min_workspace(rows)
+        assert size(rows, rows, H, D, ctx) >= fixed + rows * H * (-(-ctx // 64)) * (D + 2) * 4
+    assert size(1, 400, 8, 64, 1500) < size(1, 400, 8, 64, 4000)
+
+
 def test_reads_plan_names_the_short_decode_shapes():
     """The host-only rule for which runs read no plan: one query per sequence,
     a context bound <= 2048, head_dim 16/32/48/64, 1/2/4/8 query heads per KV

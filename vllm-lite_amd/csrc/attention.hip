@@ -3294,26 +3294,42 @@ extern "C" size_t vl_paged_attention_workspace_size(int num_seqs, int num_tokens
   if (num_seqs < 0 || num_tokens < 0 || num_heads <= 0 || head_dim <= 0) return 0;
   const int64_t S = num_seqs, H = num_heads;
   const int64_t ctx = max_context_len > 0 ? max_context_len : 1;
-  // multi-query rows split into partitions of kPart0 tokens or more (at most 64)
+  // Rows every partition could take: split short queries in parts of kPart0
+  // tokens or more (at most kMaxParts of them: contexts of 8192 tokens at that
+  // length), with their arrival counters (at most one row per query row);
+  // decode ranges of 64 tokens or more, with one counter per KV head.
+  constexpr int64_t kMaxParts = 128;
   const int64_t split_tokens = num_tokens < S * kSplitMaxQ ? num_tokens : S * kSplitMaxQ;
-  int64_t parts = std::min<int64_t>(std::max<int64_t>(cdiv64(ctx, kPart0), 1), 64);
-  // (and a split sequence's arrival counters, at most one row per query row)
-  const int64_t rows_tile = parts > 1 ? split_tokens * H * (parts + 1) : 0;
-  // decode ranges: as short as 64 tokens for small batches, at most a few
-  // items per resident workgroup (plus one short range per sequence) and at
-  // most kRangeMax (2048) tokens long otherwise
-  const int64_t rows_fast =
-      std::min<int64_t>(S * H * cdiv64(ctx, 1 << kRangeMinLog2),
-                        4 * kItemsPerWg * (int64_t)decode_grid() +
-                            S * H * (cdiv64(ctx, kRangeMax) + 1));
-  // split fp32 chunks: sum q H np <= 2 sum q H c / P2 (np >= 2 parts), with P2
-  // >= sum c nrb Hkv / (items aimed for) and q H <= kTileRows nrb Hkv; twice
-  // that covers the arrival counters and rounding
-  const int64_t rows_chunk =
-      ctx > kChunkPart ? std::min<int64_t>(4ll * kTileRows * kChunkItemsPerCu * vl_num_cus(),
-                                           2 * num_tokens * H * (cdiv64(ctx, kChunkPart) + 1))
-                       : 0;
-  const int64_t rows = std::max(rows_tile + rows_chunk, rows_fast);
+  const int64_t parts = cdiv64(ctx, kPart0);
+  const int64_t rows_tile = parts > 1 ? split_tokens * H * (std::min(parts, kMaxParts) + 1) : 0;
+  const int64_t ranges = S * H * (cdiv64(ctx, 1 << kRangeMinLog2) + 1);
+  // What the plan takes at most, from the items it aims for. Partition length P
+  // leaves at most `target` (KV head, 64-row block, partition) items but for one
+  // partition per row, so sum q H np <= kTileRows target + sum q H.
+  const int64_t tile_target =
+      (bf16_tile_shape(VL_DTYPE_BF16, head_dim) ? kTileItemsPerWg : kTileItemsPerWgF32) *
+      (int64_t)tile_grid();
+  const int64_t need_tile =
+      std::min(split_tokens * H * (parts + 1), kTileRows * tile_target + 2 * split_tokens * H);
+  // decode ranges: a few per resident workgroup (plus one short range per
+  // sequence), at most kRangeMax tokens long
+  const int64_t need_ranges = std::min(
+      ranges, kFRep * kItemsPerWg * (int64_t)decode_grid() + S * H * (cdiv64(ctx, kRangeMax) + 1));
+  // fp32 chunks: np >= 2 parts of P2 >= sum c nrb Hkv / items keys each (rounded
+  // down), so sum q H np <= 2 sum q H c / P2, and q H <= kTileRows nrb Hkv; their
+  // counters are fewer than q H / 8. (bf16 head dims 64 and 128 cut no chunk, but
+  // the type is not known here: 0 to 57 MB at head_dim 128.)
+  const int64_t need_chunk =
+      num_tokens > kSplitMaxQ && ctx > kChunkPart
+          ? std::min<int64_t>((2 * kTileRows + 2) * kChunkItemsPerCu * (int64_t)vl_num_cus() +
+                                  num_tokens * H / 8,
+                              num_tokens * H * (cdiv64(ctx, kChunkPart) + 1))
+          : 0;
+  const bool may_be_fast = head_dim == kFD && H % (4 * kFRep) == 0;  // bf16, or else fp32 chunks
+  const int64_t need =
+      std::min(num_tokens * H * (parts + 1),
+               need_tile + std::max(need_chunk, may_be_fast ? need_ranges : 0));
+  const int64_t rows = std::min(std::max(rows_tile, need_ranges) + need_chunk, need);
   return fixed_bytes(num_seqs) + (size_t)rows * row_bytes(head_dim);
 }
 
