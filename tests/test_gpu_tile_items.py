@@ -206,3 +206,18 @@ def test_a_value_row_that_is_not_finite_reaches_only_queries_that_see_it(dtype, 
     assert not np.isfinite(got[sees, heads, d0]).any()
     got[sees, heads, d0] = want[sees, heads, d0]
     check(got, want, dtype)
+
+
+def test_a_tight_workspace_cuts_chunks_into_fewer_parts():
+    """Room for about half of the parts the plan aims for: the chunk is cut into
+    longer ones (its sums run in another order than uncut), not left whole."""
+    H, Hkv, D = 2, 1, 64
+    b = make_batch([(64, 4096)], H, Hkv, D, 16, seed=7)
+    fixed = ops().lib().vl_paged_attention_min_workspace(1)
+    row = (D + 2) * 4 + 16  # a partial row: D floats, its max and sum, a range descriptor
+    parts = 4096 // 256
+    full, half, one = (run_attention(b, "f32", ws_bytes=fixed + n * (64 * H + 16) * row)
+                       for n in (parts, parts // 2, 0))
+    for got in (full, half, one):
+        check(got, expected(b, "f32"), "f32")
+    assert not np.array_equal(full, half) and not np.array_equal(half, one)

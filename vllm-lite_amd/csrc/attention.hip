@@ -63,6 +63,8 @@ constexpr int kPart0 = 1 << kPart0Log2;  // first partition length tried by the 
 // about this many items per compute unit, but not below kChunkPart keys each
 constexpr int kChunkItemsPerCu = 3;
 constexpr int kChunkPart = 256;
+// chunks are left whole when their partials do not fit with parts this long
+constexpr int kChunkPartMax = 1 << 14;
 constexpr float kLog2e = 1.4426950408889634f;
 
 // bandwidth-kernel shape
@@ -458,8 +460,8 @@ __device__ __forceinline__ int bucket_add(int* h, int key, int hot) {
 // items, i.e. a few per resident workgroup: longer ranges mean fewer split
 // partials to write and merge, shorter ones keep every CU busy) and the
 // multi-query partition length P (the smallest power of two from kPart0 that
-// leaves about tile_target items), doubling both until the split partials fit
-// the workspace. Then writes per-sequence offsets and the order
+// leaves about tile_target items), and the part length of fp32 chunks, doubling
+// the last, then both others, until the split partials fit the workspace. Then writes per-sequence offsets and the order
 // in which the shorter last ranges are handed out: longest first, after all
 // full ranges, so the kernel ends on its smallest items. The sequences with
 // 32-row tile items are ordered the same way, by context length, longest
@@ -535,8 +537,8 @@ __global__ void __launch_bounds__(kPlanThreads) plan_kernel(
     });
     plan_sum(need, red1[it & 1]);
     if (need[0] <= (unsigned long long)cap_rows || (n.lp >= kMaxLen && n.lr >= kMaxLen)) break;
-    if (n.p2 != kNoSplit)
-      n.p2 = kNoSplit;  // the chunks' partials do not fit beside the others: leave them whole
+    if (n.p2 != kNoSplit)  // longer parts of the chunks first, at last none
+      n.p2 = n.p2 < kChunkPartMax ? 2 * n.p2 : kNoSplit;
     else
       n.lp = min(n.lp + 1, kMaxLen), n.lr = min(n.lr + 1, kMaxLen);
   }
