@@ -38,6 +38,29 @@ def test_ctypes_signatures_cover_the_header():
     assert sorted(SIGNATURES) == declared()
 
 
+def test_a_stale_library_is_reported_as_one(monkeypatch):
+    """A library of another ABI revision, or one built before an entry point
+    was added: a RuntimeError that says to rebuild, not an AttributeError."""
+    from types import SimpleNamespace
+    from vllmlite_amd import ops
+
+    def library(version, names):
+        lib = SimpleNamespace(vl_abi_version=lambda: version)
+        for n in names:
+            if not hasattr(lib, n):
+                setattr(lib, n, lambda *a: 0)
+        return lib
+
+    names = [n for n in ops.SIGNATURES if n != "vl_linear_rows_deep"]
+    monkeypatch.setattr(ops, "_LIB", None)
+    monkeypatch.setattr(ops.os.path, "exists", lambda p: True)
+    for version, has, says in ((ops.ABI_VERSION - 1, names[:3], "ABI"),
+                               (ops.ABI_VERSION, names, "vl_linear_rows_deep")):
+        monkeypatch.setattr(ops.ctypes, "CDLL", lambda *a, **k: library(version, has))
+        with pytest.raises(RuntimeError, match=f"{says}.*rebuild"):
+            ops.lib()
+
+
 def test_no_compute_without_gpu_needed_for_queries():
     """Size queries are host-only and callable without a device."""
     from vllmlite_amd.build import LIB_PATH

@@ -106,13 +106,15 @@ def lib() -> ctypes.CDLL:
                 f"HIP library not built: {LIB_PATH} is missing "
                 "(run `python -m vllmlite_amd.build` or __graft_entry__.build())")
         handle = ctypes.CDLL(LIB_PATH, mode=ctypes.RTLD_GLOBAL)
+        stale = f"these bindings need ABI {ABI_VERSION}: rebuild the library"
+        if handle.vl_abi_version() != ABI_VERSION:
+            raise RuntimeError(f"{LIB_PATH} has ABI {handle.vl_abi_version()}, {stale}")
         for name, (res, args) in SIGNATURES.items():
-            fn = getattr(handle, name)
+            fn = getattr(handle, name, None)
+            if fn is None:  # built before the entry point was added
+                raise RuntimeError(f"{LIB_PATH} has no {name}, {stale}")
             fn.restype = res
             fn.argtypes = args
-        if handle.vl_abi_version() != ABI_VERSION:
-            raise RuntimeError(f"{LIB_PATH} has ABI {handle.vl_abi_version()}, these bindings "
-                               f"need {ABI_VERSION}: rebuild the library")
         _LIB = handle
     return _LIB
 
