@@ -565,7 +565,8 @@ def e2e_leg(name="mixed", repeat=3, cpu=True):
            "output_tok_per_s": round(toks / wall, 1), "wall_s": round(wall, 4),
            "steps": steps, "us_per_step": round(wall / steps * 1e6, 1), "output_tokens": toks}
     fl = mix_floor(cfg, name)
-    n_launch = mc_layers(cfg) * (4 if runner._fused_wo else 5) + 1
+    wo_fused = runner.wo_in_attention(cfg.scheduler.max_seqs)
+    n_launch = mc_layers(cfg) * (4 if wo_fused else 5) + 1
     lf = launch_floor_us(n_launch)
     out["roofline"] = {
         "bound": "hbm (weights + K/V per step at 8 TB/s; the steps are launch- and "
@@ -582,7 +583,7 @@ def e2e_leg(name="mixed", repeat=3, cpu=True):
                          "resolves the previous step's ids, reads its indices from the step's "
                          "pinned record and copies the record to the device), attention"
                          + (" with wo (one partial row per KV head), residual+norm+gate|up+SwiGLU"
-                            if runner._fused_wo else ", wo+residual, norm+gate|up+SwiGLU")
+                            if wo_fused else ", wo+residual, norm+gate|up+SwiGLU")
                          + ", down+residual; then lm_head with each row's argmax")}
     if fork:
         out["cow_pairs"] = pairs

@@ -569,3 +569,22 @@ def test_steps_from_rotating_worker_threads():
         finally:
             for p in pools:
                 p.shutdown()
+
+
+@pytest.mark.parametrize("heads,kv_heads,seqs,inside", [(8, 4, 4, True), (8, 4, 16, True),
+                                                        (8, 4, 17, False), (8, 8, 4, False),
+                                                        (4, 2, 32, True)])
+def test_wo_in_attention_names_the_launches_a_decode_step_takes(heads, kv_heads, seqs, inside):
+    """wo_in_attention (which the benchmark's launch count asks) against the
+    path the decode steps of that many sequences take: by the rows of their
+    bucket, so never with 8 KV heads."""
+    from vllmlite_amd.hip_runner import HipRunner
+    cfg = small_cfg(max_seqs=seqs)
+    cfg.model.n_heads, cfg.model.n_kv_heads, cfg.model.d_model = heads, kv_heads, 16 * heads
+    runner = HipRunner(cfg.model, cfg.cache)
+    taken = []
+    real = runner._forward_decode_wo
+    runner._forward_decode_wo = lambda s, *a: (taken.append(s.Sb), real(s, *a))
+    eng = LLMEngine(cfg, runner=runner)
+    run(eng, [f"request {i}" for i in range(seqs)], max_tokens=3)
+    assert runner.wo_in_attention(seqs) == inside == bool(taken)

@@ -65,12 +65,14 @@ from .runner import ModelRunner
 FUSED_ROWS_MAX = 1024
 # decode steps with wo inside the attention launch (one partial row per KV
 # head and row, summed again by every workgroup of gate|up): up to this many
-# partial rows, and up to this d_model (the wo columns an attention workgroup
-# multiplies by). Per step, fused against wo in a launch of its own, rows x KV
-# heads: d_model 384, 16 x 4 190 and 197 us, 16 x 8 198 and 199, 32 x 4 229 and
-# 223, 32 x 8 253 and 231; d_model 256, 16 x 2 177 and 200, 32 x 2 206 and 213,
-# 16 x 8 184 and 182, 32 x 4 208 and 207; d_model 512 (d_ff 2048), 16 x 4 238 and
-# 229, 4 x 8 245 and 216, 32 x 8 376 and 346
+# partial rows, counted in the step's bucket (16 rows or more, so at most 4 KV
+# heads), and up to this d_model (the wo columns an attention workgroup
+# multiplies by). Per step, fused against wo in a launch of its own, bucket
+# rows x KV heads: d_model 384, 16 x 4 190 and 197 us, 16 x 8 198 and 199,
+# 32 x 4 229 and 223, 32 x 8 253 and 231; d_model 256, 16 x 2 177 and 200,
+# 32 x 2 206 and 213, 16 x 8 184 and 182, 32 x 4 208 and 207; d_model 512 (d_ff
+# 2048), 16 x 4 238 and 229, 32 x 8 376 and 346 (nothing measured between 384
+# and 512)
 FUSED_WO_PARTS = 64
 FUSED_WO_D_MODEL = 384
 # execute() writes up to this many logits to the pinned host buffer by a kernel
@@ -353,8 +355,9 @@ class HipRunner(ModelRunner):
         # they select the short-decode kernel, which needs no plan
         self._short_decode = not ops.paged_attention_reads_plan(
             self.H, self.Hkv, self.hd, self.block_size, 1, mc.max_seq_len)
-        # decode steps with wo inside the attention launch (vl_decode_attention_wo)
-        self._fused_wo = (self._short_decode and self._fused_rows and self.Hkv in (1, 2, 4, 8)
+        # decode steps may have wo inside the attention launch
+        # (vl_decode_attention_wo; wo_in_attention says which)
+        self._fused_wo = (self._short_decode and self._fused_rows and self.Hkv in (1, 2, 4)
                           and mc.d_model <= FUSED_WO_D_MODEL and fused_wo)
 
     def __del__(self):
@@ -375,6 +378,11 @@ class HipRunner(ModelRunner):
     @property
     def cache_bytes(self) -> int:
         return (self.cache_k.numel() + self.cache_v.numel()) * self.cache_k.element_size()
+
+    def wo_in_attention(self, rows: int) -> bool:
+        """Whether a decode step of this many sequences runs its output projection
+        in the attention launch (four launches per layer, else five)."""
+        return self._fused_wo and _bucket(rows, 16) * self.Hkv <= FUSED_WO_PARTS
 
     def execute(self, out) -> Tuple[np.ndarray, List[Tuple[int, int]]]:
         with torch.cuda.device(self.device), torch.cuda.stream(self.stream):
@@ -693,7 +701,7 @@ class HipRunner(ModelRunner):
         launch (one partial row per KV head) and the residual add in gate|up's
         prologue: four launches per layer."""
         W, Tb, Rb = self.w, s.Tb, s.Rb
-        if s.decode and self._fused_wo and Tb * self.Hkv <= FUSED_WO_PARTS:
+        if s.decode and self.wo_in_attention(Tb):
             self._forward_decode_wo(s, x, q, act, lidx, qsl, lens, bt, ids_host, rec_host)
             return
         pos = self._meta[s.pos:s.pos + Tb]
