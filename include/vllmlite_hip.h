@@ -235,10 +235,9 @@ int vl_rope_and_cache(const float* qkv, int64_t qkv_stride, float* q_out, void* 
                       int kv_layout, int block_size, void* stream);
 
 /*
- * K6 fp32 projections of the TinyLlama forward for at most 16 token rows
- * (the decode steps), with their neighbours fused: f(x) = x, or when
- * norm_weight != NULL the RMSNorm of each row of x times norm_weight (as
- * vl_rms_norm computes it), then by mode
+ * K6 fp32 projections of the TinyLlama forward, with their neighbours fused:
+ * f(x) = x, or when norm_weight != NULL the RMSNorm of each row of x times
+ * norm_weight (as vl_rms_norm computes it), then by mode
  *   VL_LINEAR_STORE       out = f(x) @ W           (q/k/v: model.py:96-101;
  *                                                  lm_head: model.py:119-120)
  *   VL_LINEAR_ACCUMULATE  out += f(x) @ W          (the residual adds,
@@ -254,11 +253,13 @@ int vl_rope_and_cache(const float* qkv, int64_t qkv_stride, float* q_out, void* 
  * tiles, then the up tiles; weight_stride unused; 16-byte aligned; inside a
  * tile element (k, m), k = 16g + 4j + s, at flat position 256g + 4(16j + m) +
  * s, so each lane's operands of 4 MFMA steps are one 16-byte load, as are
- * the x elements they meet; norm_weight, when given, 16-byte aligned). out [rows, n]; out must not overlap x. rows <= 16 * 65535
- * (a workgroup per 16 columns and 16 rows, or 2 or 4 row tiles in turn on large
- * grids; built for the <= 16 rows of a decode step, where one row tile does
- * it), k a multiple of 16, k <= 1024.
- * fp32 throughout.
+ * the x elements they meet; norm_weight, when given, 16-byte aligned).
+ * out [rows, n]; out must not overlap x. rows <= 16 * 65535, k a multiple of
+ * 16, k <= 1024. fp32 throughout. Few rows (the <= 16 of a decode step first
+ * of all) run a workgroup per 16 columns and 4 or 16 rows; tiled weights from
+ * a grid of one 32-row x 64-column workgroup per compute unit on run 32- or
+ * 64-row workgroups. The two sum k in different orders, so a row's result is
+ * the same bits for every row count on one side of that line, not across it.
  */
 int vl_linear_rows(float* out, int64_t out_stride, const float* x, int64_t x_stride,
                    const int32_t* row_index, const float* weight, int64_t weight_stride,

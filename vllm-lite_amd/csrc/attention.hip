@@ -23,11 +23,11 @@
 //           dim is a multiple of 16 up to 128 and the block size a power of
 //           two, else to the generic kernel (one wavefront per (sequence,
 //           query, head, partition): 24 decodes + 2 chunks at head_dim 80
-//           took 784 us there, 66 on widened fp32 tiles); a batch holding both kinds runs in the one step
-//           kernel. Split sequences are merged (max-rescaled log-sum-exp)
-//           by the last workgroup to finish a partition of them, in the
-//           bandwidth, tile and step kernels, and by the combine kernel
-//           after the generic one.
+//           took 784 us there, 66 on widened fp32 tiles); a batch holding
+//           both kinds runs in the one step kernel. Split sequences are
+//           merged (max-rescaled log-sum-exp) by the last workgroup to finish
+//           a partition of them, in the bandwidth, tile and step kernels,
+//           and by the combine kernel after the generic one.
 //
 // Softmax runs in the base-2 domain: scores are pre-multiplied by
 // scale * log2(e) and exponentiated with exp2, which is the same function.
@@ -461,9 +461,9 @@ __device__ __forceinline__ int bucket_add(int* h, int key, int hot) {
 // partials to write and merge, shorter ones keep every CU busy) and the
 // multi-query partition length P (the smallest power of two from kPart0 that
 // leaves about tile_target items), and the part length of fp32 chunks, doubling
-// the last, then both others, until the split partials fit the workspace. Then writes per-sequence offsets and the order
-// in which the shorter last ranges are handed out: longest first, after all
-// full ranges, so the kernel ends on its smallest items. The sequences with
+// the last, then both others, until the split partials fit the workspace. Then
+// writes per-sequence offsets and the order in which the shorter last ranges
+// are handed out: longest first, after all full ranges, so the kernel ends on its smallest items. The sequences with
 // 32-row tile items are ordered the same way, by context length, longest
 // first (their row blocks are handed out last block first, so within a
 // sequence too the items come longest first). Every thread owns a contiguous
@@ -566,8 +566,7 @@ __global__ void __launch_bounds__(kPlanThreads) plan_kernel(
   // (32 fp32 MFMA cycles per 16 x 16 x 4 product) with one-tile decode items,
   // and the chunk items have to start first.
   auto split_items = [&](const SeqWork& w) -> int64_t {
-    if (!lpt) return w.tile;
-    // (np is 1 for most: no division there)
+    // (np is 1 for most: no division there; without lpt there are no tile items)
     return wide && w.np > 1 ? w.tile / w.np * (w.np - 1) : 0;
   };
   auto last_key = [&](int q, int c, const SeqWork& w) {
@@ -990,12 +989,6 @@ struct alignas(16) TileLds<float, D, RW> {
   int last;  // the item's workgroup arrived last among its row block's partitions
 };
 
-__device__ __forceinline__ uint32_t pack_bf16x2(float lo, float hi) {
-  return (uint32_t)f32_to_bf16(lo) | ((uint32_t)f32_to_bf16(hi) << 16);
-}
-
-
-
 // threadIdx.x, with kOpaque through an opaque move: values an item derives
 // from it are then recomputed per item instead of being hoisted out of a
 // persistent kernel's item loop, where they would stay live across the other
@@ -1008,8 +1001,9 @@ __device__ __forceinline__ int item_tid() {
 }
 
 // Kernel parameters shared by the tile and decode items: the batch, the
-// plan's per-sequence arrays and the decode items' range descriptors. They stay plain restrict-qualified kernel parameters so that the
-// compiler reads the plan's arrays with scalar loads. K/V are not restrict:
+// plan's per-sequence arrays and the decode items' range descriptors. They
+// stay plain restrict-qualified kernel parameters so that the compiler reads
+// the plan's arrays with scalar loads. K/V are not restrict:
 // restrict-qualified loads are treated as invariant and may be scheduled past
 // the compiler barriers that batch them.
 #define VL_ATTN_PARAMS(T) VL_ATTN_PARAMS_KV(T, T)
@@ -1111,7 +1105,7 @@ __device__ __forceinline__ void dev_store16(__amdgpu_buffer_rsrc_t r, uint32_t o
 // per wavefront at a time with 8-byte loads, and shuffles for the row's max
 // and sum, took 26 of the 55 us of one 400-query fp32 chunk (4 partitions).
 constexpr int kMergeFew = 8;
-template <typename T, int D, int kWv, bool kLoose = false, int kFew = kMergeFew>
+template <typename T, int D, int kWv, bool kLoose = false>
 __device__ __forceinline__ void merge_tile_rows(T* __restrict__ out, int H, int rep, int kvh,
                                                 int r_begin, int r_end, int tok0, int stride,
                                                 int np, int64_t base, const float2* ml,
@@ -1128,22 +1122,22 @@ __device__ __forceinline__ void merge_tile_rows(T* __restrict__ out, int H, int 
     const int row = (j * H + head) * stride;  // the row's first partial row, from base
     float M = -__builtin_inff(), L = 0.f;
     f32x4_t a = {0.f, 0.f, 0.f, 0.f};
-    for (int p0 = 0; p0 < np; p0 += kFew) {
-      uint64_t mv[kFew];
-      f32x4_t xv[kFew];
+    for (int p0 = 0; p0 < np; p0 += kMergeFew) {
+      uint64_t mv[kMergeFew];
+      f32x4_t xv[kMergeFew];
 #pragma unroll
-      for (int u = 0; u < kFew; ++u) {
+      for (int u = 0; u < kMergeFew; ++u) {
         const int p = min(p0 + u, np - 1);
         mv[u] = __hip_atomic_load(mlw + row + p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         xv[u] = dev_load16(pb, ((uint32_t)(row + p) * D + 4 * ch) * 4);
       }
       float Mn = M;
 #pragma unroll
-      for (int u = 0; u < kFew; ++u) Mn = fmaxf(Mn, lo_f(mv[u]));  // repeats change nothing
+      for (int u = 0; u < kMergeFew; ++u) Mn = fmaxf(Mn, lo_f(mv[u]));  // repeats change nothing
       const float alpha = M == -__builtin_inff() ? 0.f : exp2_fast(M - Mn);
       L *= alpha, a *= alpha, M = Mn;
 #pragma unroll
-      for (int u = 0; u < kFew; ++u) {
+      for (int u = 0; u < kMergeFew; ++u) {
         if (p0 + u >= np) break;  // uniform
         const float m = lo_f(mv[u]);
         const float w = m != -__builtin_inff() ? exp2_fast(m - Mn) : 0.f;

@@ -2,18 +2,19 @@
 // and the residual add or SwiGLU gate after them fused in
 // (vllmlite/model.py:96-101, 114, 116-117, 119-120). Built for few token rows
 // (the decode steps: at most 16, one row tile), and taking any number of rows
-// as 16-row tiles (the prefill steps); on large grids a workgroup takes 2 or 4
-// row tiles in turn, so that its weights serve all of them.
+// as 16-row tiles; on large grids a workgroup takes 2 or 4 row tiles in turn,
+// so that its weights serve all of them. Many rows over tiled weights (the
+// prefill steps) have a kernel of their own, linear_tile_kernel.
 //
-// One workgroup computes 16 rows x 16 output columns: its kLinWaves (8)
-// wavefronts split K into contiguous ranges on v_mfma_f32_16x16x4f32, each
-// loading its rows of x and its weights straight into operand registers (all
-// loads in flight at once, no LDS stage); the RMSNorm is applied as a per-row
-// scale after the product, so the partial tiles and sums of squares meet in
-// LDS behind one barrier and are summed in wavefront order. These kernels run
-// on few workgroups at <= 16 rows, where the dependent phases of a workgroup
-// (not the bytes) set the time: an empty kernel in a graph takes 1.9 us, one
-// that loads 40 KB per workgroup 2.3 us.
+// linear_rows_kernel: one workgroup computes 16 rows x 16 output columns: its
+// kLinWaves (8) wavefronts split K into contiguous ranges on
+// v_mfma_f32_16x16x4f32, each loading its rows of x and its weights straight
+// into operand registers (all loads in flight at once, no LDS stage); the
+// RMSNorm is applied as a per-row scale after the product, so the partial
+// tiles and sums of squares meet in LDS behind one barrier and are summed in
+// wavefront order. It runs on few workgroups at <= 16 rows, where the
+// dependent phases of a workgroup (not the bytes) set the time: an empty
+// kernel in a graph takes 1.9 us, one that loads 40 KB per workgroup 2.3 us.
 //
 // Weights come row-major ([k, n] at a row stride) or as 16-column tiles
 // ([ceil(n/16), k, 16], the columns past n zero): a workgroup's 16 columns
@@ -492,8 +493,9 @@ __global__ void __launch_bounds__(64 * kTileWaves) linear_tile_kernel(
                                                       (int64_t)(live ? ct : 0) * K * kCols) + lane;
   const int ng = K / 16, nchunk = (K + kTileK - 1) / kTileK;
   float4 px[RS], pg, wv[kSlices][kG];
-  // loads of chunk c; columns past K repeat the last 16-k group (their weights
-  // are zeroed below)
+  // loads of chunk c; past K both repeat the last 16-k group, and x is staged as
+  // zeros there (so a weight of that group that is not finite adds a NaN, as the
+  // kernel above does where its last wavefronts have fewer groups)
   auto load_x = [&](int c) {
     const int k = min(c * kTileK + sk, K - 4);
 #pragma unroll

@@ -156,10 +156,10 @@ def flatten_scheduled(out, block_size: int, max_seq_len: int) -> Flattened:
 
 
 def fused_rows_supported(mc) -> bool:
-    """Steps of up to FUSED_ROWS_MAX token rows run the fused projection
-    kernels (vl_linear_rows, vl_qkv_rope_cache), which need d_model and d_ff to be
-    multiples of 16 within their K limits; other shapes take the GEMM path for
-    every step and keep no tiled weight copies."""
+    """Whether every projection has a shape of vl_linear_rows / vl_qkv_rope_cache
+    (d_model and d_ff multiples of 16 within their K limits): what the
+    one-launch decode step asks for. rows_kernels_supported decides whether
+    steps of up to FUSED_ROWS_MAX rows run the fused projection kernels."""
     return (mc.d_model % 16 == 0 and mc.d_ff % 16 == 0 and mc.d_model <= 512
             and mc.d_ff <= 1024)
 
@@ -167,7 +167,8 @@ def fused_rows_supported(mc) -> bool:
 def rows_kernels_supported(mc) -> bool:
     """Whether every projection of the model has a fused kernel: the shapes of
     fused_rows_supported, and those whose down projection is deeper than
-    vl_linear_rows takes (vl_linear_rows_deep)."""
+    vl_linear_rows takes (vl_linear_rows_deep). Other models take the GEMM path
+    for every step and keep no tiled weight copies."""
     return (mc.d_model % 16 == 0 and mc.d_ff % 16 == 0 and mc.d_model <= 512
             and mc.d_ff <= ops.LINEAR_DEEP_K)
 
