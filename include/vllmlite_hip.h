@@ -256,10 +256,10 @@ int vl_rope_and_cache(const float* qkv, int64_t qkv_stride, float* q_out, void* 
  * the x elements they meet; norm_weight, when given, 16-byte aligned).
  * out [rows, n]; out must not overlap x. rows <= 16 * 65535, k a multiple of
  * 16, k <= 1024. fp32 throughout. Few rows (the <= 16 of a decode step first
- * of all) run a workgroup per 16 columns and 4 or 16 rows; tiled weights from
- * a grid of one 32-row x 64-column workgroup per compute unit on run 32- or
- * 64-row workgroups. The two sum k in different orders, so a row's result is
- * the same bits for every row count on one side of that line, not across it.
+ * of all) run a workgroup per 16 columns and 4 or 16 rows; many rows of tiled
+ * weights (32-row x 64-column workgroups for every compute unit) run 32- or
+ * 64-row workgroups. The two sum k in different orders: a row's result is the
+ * same bits for every row count that takes the same one, not for all.
  */
 int vl_linear_rows(float* out, int64_t out_stride, const float* x, int64_t x_stride,
                    const int32_t* row_index, const float* weight, int64_t weight_stride,

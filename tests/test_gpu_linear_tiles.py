@@ -1,5 +1,5 @@
-"""The projections of many rows (linear_tile_kernel, chosen from a grid of one
-32-row workgroup per compute unit) and the deep down projection, against
+"""The projections of many rows (linear_tile_kernel, chosen by how its 32-row
+workgroups fill the compute units) and the deep down projection, against
 float64 NumPy, and a model that needs both against the oracle runner."""
 
 import numpy as np
@@ -18,15 +18,61 @@ def _dev(a):
     return torch.from_numpy(np.ascontiguousarray(a)).cuda()
 
 
-def _rows_per_workgroup(rows, n):
+def _rows_per_workgroup(rows, n, k, mode="store", norm=False):
     """What the dispatch takes for this many rows and columns (linear.hip:
     takes_tiles, launch_tiles): 64- or 32-row workgroups of
     linear_tile_kernel, or 0 (linear_rows_kernel)."""
     cus = torch.cuda.get_device_properties(0).multi_processor_count
-    cb = -(-(-(-n // 16)) // 4)
-    if cb * -(-rows // 32) < cus:
+    ntile, row_tiles = -(-n // 16), -(-rows // 16)
+    cb = -(-ntile // 4)
+    grid, swiglu = cb * -(-rows // 32), mode == "swiglu"
+    rounds = -(-grid // cus)
+    nsub = 1
+    while nsub < 4 and ntile * -(-row_tiles // (2 * nsub)) >= 2 * cus:
+        nsub *= 2
+    groups = -(-row_tiles // nsub)
+    wgs = ntile * groups
+    whole = -(-wgs // cus) - 1
+    load = whole * nsub + (row_tiles - (groups - 1) * nsub if wgs - whole * cus <= ntile else nsub)
+    if grid < cus:
         return 0
-    return 64 if cb * -(-rows // 64) >= 2 * cus else 32
+    if swiglu and 320 < k <= 384:
+        tiles = rounds > 3 or (rounds > 1 and load > 7 * rounds)
+    else:
+        close = 256 < k <= 512 if swiglu else not norm and k <= 1024
+        tiles = rounds != 2 or not close or load >= 12
+    return 0 if not tiles else 64 if cb * -(-rows // 64) >= 2 * cus else 32
+
+
+@pytest.mark.parametrize("rows,k,n,mode,wg_rows",
+                         [(512, 384, 1024, "swiglu", 0), (800, 384, 1024, "swiglu", 0),
+                          (896, 384, 1024, "swiglu", 32), (1280, 336, 1024, "swiglu", 0),
+                          (512, 320, 1024, "swiglu", 32), (544, 320, 1024, "swiglu", 0),
+                          (544, 256, 1024, "swiglu", 32), (576, 512, 1024, "swiglu", 32),
+                          (288, 512, 2048, "swiglu", 0), (289, 512, 2048, "swiglu", 0),
+                          (305, 512, 2048, "swiglu", 32), (1000, 512, 512, "store", 32),
+                          (1056, 512, 512, "store", 0), (1056, 512, 512, "norm", 32),
+                          (768, 384, 768, "store", 32), (1376, 384, 384, "accumulate", 0),
+                          (1376, 1024, 384, "accumulate", 0),
+                          (1400, 1024, 384, "accumulate", 32), (1400, 384, 768, "accumulate", 32)])
+def test_which_kernel_many_rows_take(rows, k, n, mode, wg_rows):
+    """The sizes on both sides of the rule's lines. Row-major weights always run
+    linear_rows_kernel, so a tiled weight that gives its bits ran it too."""
+    norm, mode = mode == "norm", "store" if mode == "norm" else mode
+    assert _rows_per_workgroup(rows, n, k, mode, norm) == wg_rows
+    o = _ops()
+    rng = np.random.default_rng(rows + k)
+    halves = 2 if mode == "swiglu" else 1
+    x, w = _dev(rng.standard_normal((rows, k)).astype(np.float32)), _dev(
+        (0.05 * rng.standard_normal((k, halves * n))).astype(np.float32))
+    g = torch.ones(k, device="cuda") if norm else None
+    kind = {"store": o.LINEAR_STORE, "accumulate": o.LINEAR_ACCUMULATE,
+            "swiglu": o.LINEAR_SWIGLU}[mode]
+    tiled, plain = (torch.zeros(rows, n, device="cuda") for _ in range(2))
+    o.linear_rows(tiled, x, o.tile16(w, halves), g, mode=kind)
+    o.linear_rows(plain, x, w, g, mode=kind)
+    assert torch.equal(tiled, plain) == (wg_rows == 0)
+    _close(tiled.cpu().numpy(), plain.cpu().numpy())
 
 
 # 32- and 64-row workgroups, a last row block and a last column block that are
@@ -34,13 +80,13 @@ def _rows_per_workgroup(rows, n):
 @pytest.mark.parametrize("rows,k,n,mode,wg_rows",
                          [(1400, 1024, 384, "accumulate", 32), (1000, 496, 1100, "store", 32),
                           (1030, 384, 1152, "store", 32), (700, 64, 1030, "swiglu", 32),
-                          (260, 512, 2048, "swiglu", 32), (2050, 16, 520, "store", 32),
+                          (260, 512, 2048, "swiglu", 0), (2050, 16, 520, "store", 32),
                           (1024, 512, 2048, "swiglu", 64), (1000, 400, 2041, "swiglu", 64),
                           (2050, 16, 1030, "store", 64), (2050, 336, 1100, "store", 64),
                           (4111, 1024, 512, "accumulate", 64)])
 @pytest.mark.parametrize("norm", [False, True])
 def test_many_rows_over_tiled_weights(rows, k, n, mode, wg_rows, norm):
-    assert _rows_per_workgroup(rows, n) == wg_rows
+    assert _rows_per_workgroup(rows, n, k, mode, norm) == wg_rows
     o = _ops()
     rng = np.random.default_rng(rows + k + norm)
     halves = 2 if mode == "swiglu" else 1
@@ -62,8 +108,8 @@ def test_many_rows_over_tiled_weights(rows, k, n, mode, wg_rows, norm):
 @pytest.mark.parametrize("rows", [1, 16, 33, 1100, 4111])
 @pytest.mark.parametrize("k,n", [(16, 512), (1040, 40), (2048, 512)])
 def test_deep_projection(rows, k, n):
-    assert _rows_per_workgroup(rows, n) == (0 if rows < 1100 or n < 512 else
-                                            32 if rows == 1100 else 64)
+    assert _rows_per_workgroup(rows, n, k) == (0 if rows < 1100 or n < 512 else
+                                               32 if rows == 1100 else 64)
     o = _ops()
     rng = np.random.default_rng(rows + k)
     x = rng.standard_normal((rows, k)).astype(np.float32)
@@ -92,7 +138,7 @@ def test_many_rows_qkv_equals_projection_then_rope(layout, cache, rows, wg_rows)
     o = _ops()
     H, Hkv, D, k = 8, 4, 48, 384
     n = (H + 2 * Hkv) * D
-    assert _rows_per_workgroup(rows, n) == wg_rows
+    assert _rows_per_workgroup(rows, n, k, norm=True) == wg_rows
     blocks = -(-rows // 16)
     rng = np.random.default_rng(3)
     table = _dev(rng.standard_normal((261, k)).astype(np.float32))
@@ -160,7 +206,7 @@ def test_long_prompts_through_the_runner(lens, bucket):
     for f, v in dict(n_heads=8, n_kv_heads=8, d_model=512, d_ff=2048).items():
         setattr(cfg.model, f, v)
     assert bucket // 2 < sum(n + 1 for n in lens) < bucket
-    assert _rows_per_workgroup(bucket, 2048) == (64 if bucket == 1024 else 32)
+    assert _rows_per_workgroup(bucket, 2048, 512, "swiglu", True) == (64 if bucket == 1024 else 32)
     rng = np.random.default_rng(bucket)
     prompts = ["".join(chr(c) for c in rng.integers(32, 127, n)) for n in lens]
     runners = []

@@ -681,18 +681,6 @@ int launch_tiles(float* out, int64_t ldo, const float* x, int64_t ldx, const flo
   return VL_OK;
 }
 
-// Whether M rows over a tiled weight of N columns take the kernel above: from a
-// grid of one 32-row workgroup per compute unit on. Below, the 8 wavefronts
-// that linear_rows_kernel puts on each 16 x 16 output split K and finish
-// sooner: K 2048, N 512 at 512 rows (128 workgroups) 22.9 against 29.2 us, at
-// 1024 rows 41.9 against 29.6; K 512, N 2 x 2048 (SwiGLU) at 256 rows (256
-// workgroups) 20.3 against 17.2, at 2048 rows 150 against 88; K 512, N 1536 at
-// 1024 rows 32.5 against 21.4.
-inline bool takes_tiles(int M, int N) {
-  const int64_t cb = ((N + kCols - 1) / kCols + kTileWaves - 1) / kTileWaves;
-  return cb * ((M + 31) / 32) >= vl_num_cus();
-}
-
 // Row tiles per workgroup: 1 while the grid is at most one round of two
 // workgroups per CU (the kernel is latency-bound there, so tiles run side by
 // side); beyond that doubled, up to kSubMax, while the grid keeps at
@@ -704,6 +692,49 @@ inline int rows_per_workgroup(int ntile, int row_tiles) {
          (int64_t)ntile * ((row_tiles + 2 * nsub - 1) / (2 * nsub)) >= round)
     nsub *= 2;
   return nsub;
+}
+
+// linear_rows_kernel's load on the busiest compute unit, in 16 x 16 outputs: its
+// workgroups go round the units in order, so those past the last whole round
+// are of the last row group (which may have fewer row tiles) if they are no more
+// than its columns.
+inline int64_t rows_kernel_load(int M, int N) {
+  const int64_t cus = vl_num_cus();
+  const int ntile = (N + kCols - 1) / kCols, row_tiles = (M + kRowsMax - 1) / kRowsMax;
+  const int nsub = rows_per_workgroup(ntile, row_tiles);
+  const int groups = (row_tiles + nsub - 1) / nsub;
+  const int64_t wgs = (int64_t)ntile * groups, rounds = (wgs + cus - 1) / cus;
+  const bool last_group = wgs - (rounds - 1) * cus <= ntile;
+  return (rounds - 1) * nsub + (last_group ? row_tiles - (groups - 1) * nsub : nsub);
+}
+
+// Whether M rows over a tiled weight of N columns take linear_tile_kernel, by the
+// rounds its 32-row workgroups make over the compute units (all times: us per
+// launch in a graph, linear_rows_kernel and then linear_tile_kernel). Below one
+// round the 8 wavefronts that linear_rows_kernel puts on each 16 x 16 output
+// split K and finish sooner (K 2048, N 512 at 512 rows, half a round: 22.9 and
+// 32.1); from one round on a staged row and a weight load serve more products
+// (the same at 1024 rows 41.8 and 32.8, at 2048 81.8 and 49.3; K 512, N 1536 at
+// 1024 rows 31.7 and 21.4; K 512, N 2 x 2048, SwiGLU, at 256 rows 19.5 and 17.2, at
+// 512 36.9 and 26.7). A second round costs half of the first however few
+// workgroups it has, so linear_rows_kernel keeps sizes just past one round, where
+// its own last round is short too (a load below 12: K 384, N 384 at 1376 rows 10.2
+// and 11.5, at 1408 12.0 and 11.7; K 1024, N 384 at 1376 23.1 and 25.4; K 512, N 512 at
+// 1056 12.6 and 14.7; SwiGLU K 512, N 2 x 2048 at 288 24.1 and 26.2), except where it
+// is further behind: K above 1024 (K 2048, N 512 at 1056 52.1 and 48.2), with a norm
+// (K 1024, N 1024 at 544 32.2 and 26.6) and SwiGLU of K up to 256, which it pads to
+// 384 (N 2 x 1024 at 544 17.3 and 16.0). SwiGLU at K just below that depth is its best
+// case (K 384, N 2 x 1024 at 512, 576, 800, 1024, 1280, 1536 rows 13.2, 19.6, 21.0, 24.5,
+// 30.6, 36.0 and 13.7, 21.2, 21.6, 21.7, 31.9, 32.5).
+inline bool takes_tiles(int M, int N, int K, bool norm, bool swiglu) {
+  const int64_t cus = vl_num_cus();
+  const int64_t cb = ((N + kCols - 1) / kCols + kTileWaves - 1) / kTileWaves;
+  const int64_t grid = cb * ((M + 31) / 32), rounds = (grid + cus - 1) / cus;
+  if (grid < cus) return false;
+  if (swiglu && K > 320 && K <= 384)
+    return rounds > 3 || (rounds > 1 && rows_kernel_load(M, N) > 7 * rounds);
+  const bool close = swiglu ? K > 256 && K <= 512 : !norm && K <= 1024;
+  return rounds != 2 || !close || rows_kernel_load(M, N) >= 12;
 }
 
 // Rows per row tile. A step of at most 16 rows (a decode step) runs as row
@@ -727,7 +758,7 @@ int launch(float* out, int64_t ldo, const float* x, int64_t ldx, const float* w,
            const int32_t* prev_ids = nullptr, int64_t num_prev = 0,
            const float* x_parts = nullptr, const ArgmaxOut& am = ArgmaxOut{}) {
   if constexpr (MODE != 4 && NP == 0) {
-    if (tiles && takes_tiles(M, N))
+    if (tiles && takes_tiles(M, N, K, NORM, MODE == 2))
       return launch_tiles<MODE, NORM>(out, ldo, x, ldx, w, norm_w, eps, M, K, N, st, row_index, rc,
                                       x_out, prev_ids, num_prev);
   }
