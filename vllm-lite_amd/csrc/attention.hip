@@ -32,6 +32,7 @@
 // Softmax runs in the base-2 domain: scores are pre-multiplied by
 // scale * log2(e) and exponentiated with exp2, which is the same function.
 #include <algorithm>
+#include <cfloat>
 #include <mutex>
 #include <type_traits>
 
@@ -1313,6 +1314,21 @@ __device__ __forceinline__ void tile_body(TileLds<T, D, RW>& lds, int it, int pa
         }
       }
     }
+    // The fp32 path takes a negative scale, as the generic kernel does: its sign
+    // goes into q (exactly), so that a masked score, -inf times |scale|, stays
+    // -inf and the largest score the maximum. (In a branch: a use of q here waits
+    // for it before the first tile is asked for; always multiplied, 3 decodes at
+    // head_dim 128 took 25.8 us instead of 24.1.)
+    if constexpr (!kBf16) {
+      if (scale_log2 < 0.f) {  // uniform
+#pragma unroll
+        for (int s = 0; s < kKS; ++s) qop[s] = -qop[s];
+      }
+    }
+    auto scaled = [&](float x) { return x * (kBf16 ? scale_log2 : fabsf(scale_log2)); };
+    auto exponent = [&](float x, float neg_ref) {  // scaled x - reference
+      return fmaf(x, kBf16 ? scale_log2 : fabsf(scale_log2), neg_ref);
+    };
     AccT acc[kDT];
 #pragma unroll
     for (int u = 0; u < kDT; ++u)
@@ -1554,7 +1570,7 @@ __device__ __forceinline__ void tile_body(TileLds<T, D, RW>& lds, int it, int pa
       } else {
         cmax = fmaxf(cmax, __shfl_xor(cmax, 32, 64));
       }
-      const float cm = cmax * scale_log2;
+      const float cm = scaled(cmax);
       if (__any(cm > m_run + kLazy)) {
         const float m_new = fmaxf(m_run, cm);
         const float alpha = m_new == -__builtin_inff() ? 1.f : exp2_fast(m_run - m_new);
@@ -1596,7 +1612,7 @@ __device__ __forceinline__ void tile_body(TileLds<T, D, RW>& lds, int it, int pa
       for (int t = 0; t < kST; ++t)
 #pragma unroll
         for (int r = 0; r < kCV; ++r) {
-          pr[t][r] = exp2_fast(fmaf(sc[t][r], scale_log2, neg_ref));
+          pr[t][r] = exp2_fast(exponent(sc[t][r], neg_ref));
           if constexpr (!kW) psum += pr[t][r];
         }
       if constexpr (!kW) l_part += psum;
@@ -1701,7 +1717,7 @@ __device__ __forceinline__ void tile_body(TileLds<T, D, RW>& lds, int it, int pa
         }
         cmax = fmaxf(cmax, __shfl_xor(cmax, 16, 64));
         cmax = fmaxf(cmax, __shfl_xor(cmax, 32, 64));
-        const float m_new = fmaxf(m_run, cmax * scale_log2);
+        const float m_new = fmaxf(m_run, scaled(cmax));
         const float alpha = m_new == -__builtin_inff() ? 1.f : exp2_fast(m_run - m_new);
         const float ref = m_new == -__builtin_inff() ? 0.f : m_new;
         m_run = m_new;
@@ -1710,7 +1726,7 @@ __device__ __forceinline__ void tile_body(TileLds<T, D, RW>& lds, int it, int pa
         for (int u = 0; u < kDT; ++u) acc[u] *= alpha;
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          sc[r] = exp2_fast(fmaf(sc[r], scale_log2, -ref));
+          sc[r] = exp2_fast(exponent(sc[r], -ref));
           l_part += sc[r];
         }
 #pragma unroll
@@ -1780,19 +1796,6 @@ __device__ __forceinline__ void tile_body(TileLds<T, D, RW>& lds, int it, int pa
       }
     } else {
       if (ntile > 0) prefetch(kbeg, pk, pv);
-      if constexpr (!kBf16) {
-        // The fp32 path takes any scale, as the generic kernel does: a sign goes
-        // into q (exactly; a scale of 0 makes q 0), so that a masked score, -inf
-        // times what is left of it, stays -inf and the largest score the maximum.
-        // (Here, not where q is loaded: a use there waits for q before the first
-        // tile is asked for, 3 decodes at head_dim 128 24.1 -> 25.8 us.)
-        if (!(scale_log2 > 0.f)) {  // uniform
-          const float sign = scale_log2 < 0.f ? -1.f : scale_log2;  // 0, or a NaN
-          scale_log2 = scale_log2 == 0.f ? 1.f : fabsf(scale_log2);
-#pragma unroll
-          for (int s = 0; s < kKS; ++s) qop[s] *= sign;
-        }
-      }
       for (int ti = 0; ti < ntile; ++ti) tile_step(ti, 1, pk, pv);
     }
     if constexpr (kLoose) {
@@ -1803,7 +1806,7 @@ __device__ __forceinline__ void tile_body(TileLds<T, D, RW>& lds, int it, int pa
       // that ends on a NaN computes its rows again, key by key. (Looking for
       // such elements as a tile is staged cost 2-5 % of a mixed batch.)
       bool nan = false;
-      if (kend_wg - 1 > ctx - q_len + rbase / rep) {  // uniform
+      if (kend_wg - 1 > qpos_wave_min) {  // uniform over the wavefront
 #pragma unroll
         for (int u = 0; u < kDT; ++u)
 #pragma unroll
@@ -1828,7 +1831,7 @@ __device__ __forceinline__ void tile_body(TileLds<T, D, RW>& lds, int it, int pa
           s += __shfl_xor(s, 16, 64);
           s += __shfl_xor(s, 32, 64);
           if (key > qpos) continue;
-          s *= scale_log2;
+          s = scaled(s);
           const float m_new = fmaxf(m_run, s);
           const float ref = m_new == -__builtin_inff() ? 0.f : m_new;
           const float alpha = exp2_fast(m_run - ref), p = exp2_fast(s - ref);
@@ -3103,6 +3106,10 @@ int tile_launch_grid() {
 template <typename T, int D, int RW, typename TKV = T, typename TIO = T>
 int launch_tile_d(const Args& a, const Layout& L, float sl2, hipStream_t st) {
   constexpr int kWv = RW == 32 ? 8 : 4;
+  // fp32 items multiply masked scores, -inf, by |scale|: a scale of 0 (every
+  // visible key weighs the same) goes as the smallest normal number, which
+  // leaves the exponents of scores up to 1e30 at 0
+  if (sizeof(T) == 4 && sl2 == 0.f) sl2 = FLT_MIN;
   attend_tile_kernel<T, D, RW, kWv, TKV, TIO>
       <<<tile_launch_grid<T, D, RW, kWv, TKV, TIO>(), 64 * kWv, 0, st>>>(
           VL_ATTN_LAUNCH_ARGS_KV(TIO, TKV), L.hdr, RW == 32 ? L.wide_off : L.tile_off,
