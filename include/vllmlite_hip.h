@@ -128,7 +128,9 @@ size_t vl_paged_attention_min_workspace(int num_seqs);
  * head_dim 128, 4 query heads per KV head and 16-token blocks: max 1 launches
  * only the decode kernel, min 1 with max > 1 (decodes and multi-query
  * sequences) only the one-launch step kernel, min > 1 only the multi-query
- * kernels; with a bound unknown the kernels decide on the device. Bounds that
+ * kernels; with a bound unknown the kernels decide on the device. For bf16 at
+ * head_dim 64 and 128, min > 16 leaves out the kernel of the sequences with up
+ * to 16 queries, max <= 16 that of the longer ones. Bounds that
  * do not hold leave some sequences' outputs unwritten (nothing is read or
  * written out of bounds).
  */

@@ -830,12 +830,13 @@ __global__ void __launch_bounds__(64) attend_generic_kernel(
 // bf16 uses v_mfma_f32_16x16x32_bf16 (P rounded to bf16, fp32 accumulation);
 // fp32 uses v_mfma_f32_16x16x4f32, so fp32 inputs keep fp32 products.
 //
-// The fp32 items are bound by the matrix pipe: a 64-key tile of 16 rows at
-// head_dim 64 is 128 products of 32 cycles (1.7 us at 2.4 GHz), against 0.9 us
-// for its softmax, staging and barriers. One 16-byte LDS read feeds 4 products
-// of QK^T or PV (4-byte reads at an odd row stride met 4-way bank conflicts);
-// items start longest first, and chunks are cut over the context into about
-// 3 items per compute unit, so that one long row block does not set the time.
+// The fp32 items: a 64-key tile of 16 rows at head_dim 64 is 128 products of 32
+// cycles (1.7 us at 2.4 GHz) between its softmax, staging and barriers; over the
+// launch measured below the matrix pipes are busy 32 % of the time. One 16-byte
+// LDS read feeds 4 products of QK^T or PV (4-byte reads at an odd row stride
+// met 4-way bank conflicts); items start longest first, and chunks are cut over
+// the context into about 3 items per compute unit, so that one long row block
+// does not set the time.
 // 24 decodes + 5 chunks of 300-500 queries, 8 heads of 64: 208 us before, of it
 // 201 in this kernel; 160 with the wide reads, 126 with the order and the cut,
 // 101 with the 16-byte merge (merge_tile_rows).
