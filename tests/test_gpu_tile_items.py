@@ -1,5 +1,6 @@
-"""The tile kernel's work items at the edges of their rules, against the
-oracle: fp32 query chunks cut over the context."""
+"""The tile kernel's work items at the edges of their rules, against the oracle:
+fp32 query chunks cut over the context, head dims widened to fp32 products,
+values and lengths at the limits, plans over many sequences."""
 
 import numpy as np
 import pytest
@@ -221,3 +222,15 @@ def test_a_tight_workspace_cuts_chunks_into_fewer_parts():
     for got in (full, half, one):
         check(got, expected(b, "f32"), "f32")
     assert not np.array_equal(full, half) and not np.array_equal(half, one)
+
+
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+def test_more_sequences_than_the_plan_keeps_in_lds(dtype):
+    """Over 2048 sequences the plan recomputes item counts instead of keeping
+    them: decodes, short verifies and chunks in one longest-first list."""
+    S = 2100
+    seqs = [((1, 1 + i % 97) if i % 7 else (5, 5 + i % 140)) for i in range(S)]
+    seqs[1000] = (40, 700)
+    seqs[2099] = (20, 333)
+    b = make_batch(seqs, 2, 1, 80, 16, seed=11)
+    check(run_attention(b, dtype), expected(b, dtype), dtype)
